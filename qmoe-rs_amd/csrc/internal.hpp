@@ -165,6 +165,13 @@ qmla_status launch_prefill_f32(const qmla_prefill_dims &d, const float *q_nope,
                                const float *q_rope, const float *k, const float *k_rope,
                                const float *v, float scale, int causal, float *out,
                                hipStream_t stream);
+// The f32 MFMA form of launch_prefill_f32 and the calls it takes.
+bool prefill_f32_mfma_supported(const qmla_prefill_dims &d, const float *q_nope, const float *q_rope,
+                                const float *k, const float *k_rope, const float *v, const float *out);
+qmla_status launch_prefill_f32_mfma(const qmla_prefill_dims &d, const float *q_nope,
+                                    const float *q_rope, const float *k, const float *k_rope,
+                                    const float *v, float scale, int causal, float *out,
+                                    hipStream_t stream);
 // (dn, dr, dv) combinations the bf16 MFMA prefill takes.
 bool prefill_bf16_supported(int dn, int dr, int dv);
 // Shapes whose bf16 prefill can write the context as records (below).

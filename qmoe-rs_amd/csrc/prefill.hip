@@ -130,6 +130,8 @@ qmla_status launch_prefill_f32(const qmla_prefill_dims &d, const float *q_nope, 
                                int causal, float *out, hipStream_t stream) {
   QMLA_REQUIRE(d.qk_nope + d.qk_rope <= kPfMaxQK && d.v_dim <= kPfMaxV, QMLA_ERR_UNSUPPORTED,
                "f32 prefill supports qk width <= %d and v width <= %d", kPfMaxQK, kPfMaxV);
+  if (prefill_f32_mfma_supported(d, q_nope, q_rope, k, k_rope, v, out))
+    return launch_prefill_f32_mfma(d, q_nope, q_rope, k, k_rope, v, scale, causal, out, stream);
   dim3 grid((d.seq_q + kPfRows - 1) / kPfRows, d.heads, d.batch), block(kPfThreads);
   const int vpt = (d.v_dim + 3) / 4;
   if (vpt <= 8)

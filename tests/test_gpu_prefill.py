@@ -216,3 +216,31 @@ def test_prefill_unsupported_bf16_dims_raise(qmla_gpu):
     with pytest.raises(q.QmlaError) as e:
         q.prefill_numpy(*arrs, 0.1, True, dtype=q.BF16)
     assert e.value.status == 3
+
+
+@pytest.mark.parametrize("b,h,sq,sk,off,causal,krh", [
+    (1, 1, 1, 1, 0, True, 1), (2, 3, 31, 31, 0, True, 3), (1, 2, 33, 97, 64, True, 1), (1, 3, 32, 129, 0, False, 1),
+    (1, 1, 5, 300, 200, True, 1),   # keys beyond the last row's horizon
+    (2, 8, 1030, 1030, 0, True, 1),  # blocks dealt per XCD
+    (1, 9, 1830, 40, 0, False, 9)])  # more than two blocks per CU, heads no multiple of 8
+def test_prefill_f32_mfma_edges(qmla_gpu, b, h, sq, sk, off, causal, krh):
+    """Tile remainders, block orders and scores that grow along the keys.
+    The oracle sums in f32 too: scores up to ~40 with 2^-24 per term over
+    sqrt(192) terms give each side a few 1e-6 of p, 2e-5 with the margin."""
+    arrs = inputs(b, h, sq, sk, 128, 64, 128, krh, 700 + sq)
+    arrs[2] += np.linspace(0.0, 3.0, sk, dtype=np.float32)[:, None]
+    out, _ = gpu_prefill(qmla_gpu, arrs, 192 ** -0.5, causal, q_offset=off)
+    ref = O.fused_prefill_attn(*arrs, 192 ** -0.5, causal, q_offset=off)
+    assert rel_err(out, ref) < 2e-5
+
+
+def test_prefill_f32_unaligned_tensors(qmla_gpu):
+    """Tensors that are only 4-byte aligned take the VALU kernel: same result."""
+    q = qmla_gpu
+    arrs = inputs(1, 2, 70, 70, 128, 64, 128, 1, 790)
+    dims = q.PrefillDims(1, 2, 70, 70, 128, 64, 128, 1, 0)
+    bufs = [q.DeviceBuffer.from_numpy(np.concatenate([np.zeros(1, np.float32), a.ravel()])) for a in arrs]
+    out = q.DeviceBuffer(arrs[4].nbytes + 4)
+    q.fused_prefill_attn(*[x.ptr + 4 for x in bufs], 0.1, True, dims=dims, dtype=q.F32, out=out.ptr + 4)
+    got = out.to_numpy(np.float32, (1 + arrs[4].size,))[1:].reshape(arrs[4].shape)
+    assert rel_err(got, q.prefill_numpy(*arrs, 0.1, True)) < 2e-5
