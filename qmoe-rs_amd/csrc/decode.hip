@@ -396,9 +396,19 @@ int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t
   if (cus <= 0) cus = 256;
   int per_cu = (c->dtype == QMLA_BF16 && decode_mfma_supported(d->rows, d->kv_lora_rank, d->rope_dim))
                    ? decode_mfma_blocks_per_cu(d->rows, d->kv_lora_rank, d->rope_dim)
-                   : 4;
+                   : decode_f32_blocks_per_cu(d->kv_lora_rank, d->rope_dim);
   int64_t target = (int64_t)cus * per_cu;
-  const int64_t min_tokens = 128;
+  int64_t min_tokens = 128;
+  // The f32 MFMA decode reads its 32-token tiles at 1.2 us each, so few
+  // tokens go out one tile to a piece (counting the plan's virtual tokens):
+  // 278 tokens 27.8 us at 128 a piece, 14.1 at 32; 2222 tokens 28.3 and 17.3.
+  // At most 32 rows and 64 sequences, where the partials of 256 pieces stay
+  // below 22 MB.
+  if (c->dtype == QMLA_F32 && decode_f32_mfma_supported(d->kv_lora_rank, d->rope_dim) && d->rows <= 32 &&
+      d->batch <= 64) {
+    min_tokens = 32;
+    total += (int64_t)d->batch * kDecodeF32SegTokens;
+  }
   int64_t by_work = (total + min_tokens - 1) / min_tokens;
   int64_t blocks = std::max<int64_t>(1, std::min(target, by_work));
   return (int32_t)std::min<int64_t>(blocks, kMaxPlanBlocks);
@@ -434,7 +444,8 @@ qmla_status qmla::decode_launch(const qmla_decode_dims *d, const qmla_kv_cache *
   QMLA_REQUIRE(ws != nullptr && ws_bytes >= lay.total, QMLA_ERR_WORKSPACE,
                "workspace of %zu bytes < required %zu", ws_bytes, lay.total);
   DecodePlanView plan{};
-  if (!mfma) {
+  const bool f32_mfma = !mfma && decode_f32_mfma_supported(d->kv_lora_rank, d->rope_dim);
+  if (!mfma && !f32_mfma) {
     plan = decode_plan_view(ws, d->batch, blocks);
     int64_t total = 0;
     for (int32_t i = 0; i < d->batch; ++i) total += c->h_lens[i];
@@ -461,6 +472,7 @@ qmla_status qmla::decode_launch(const qmla_decode_dims *d, const qmla_kv_cache *
   a.pending = pending;
   a.advance = advance;
   if (mfma) return launch_decode_mfma(a, s);  // decode + merge
+  if (f32_mfma) return launch_decode_f32_mfma(a, s);
   QMLA_TRY(launch_decode_f32(a, s));
   return launch_decode_merge(d->batch, d->rows, d->kv_lora_rank, plan, a.part_o, a.part_lse, out,
                              out_lse, advance ? c->d_lens : nullptr, pending, s);

@@ -97,6 +97,7 @@ struct DecodePlanView {
 // The bf16 MFMA path plans inside its kernel: instead of the plan it keeps
 // per-sequence {first slot, slot count} (int2 x batch), and its partial rows
 // are padded to a multiple of 32 (fragment-major layout, see decode_mfma).
+// The f32 MFMA path keeps that int2 table in the plan's place.
 struct DecodeWorkspace {
   size_t plan_bytes = 0;
   size_t part_o_off = 0;
@@ -135,8 +136,8 @@ struct DecodeArgs {
   float scale;
   float *out;         // [batch, rows, r]
   float *out_lse;     // [batch, rows] or null
-  DecodePlanView plan;  // f32 path
-  int2 *seq_info;       // MFMA path: [batch] {first slot, slot count}
+  DecodePlanView plan;  // VALU f32 path
+  int2 *seq_info;       // MFMA paths: [batch] {first slot, slot count}
   float *part_o;
   float *part_lse;
   int32_t blocks;
@@ -151,6 +152,15 @@ constexpr int32_t kMaxPlanBatch = 8192;
 constexpr int32_t kMaxPlanBlocks = 8192;
 qmla_status launch_decode_f32(const DecodeArgs &a, hipStream_t stream);
 qmla_status launch_decode_mfma(const DecodeArgs &a, hipStream_t stream);
+// f32 caches of these widths: decode_f32_mfma.hip (decode + merge), planned
+// in the kernel like the bf16 path.
+bool decode_f32_mfma_supported(int32_t r, int32_t dr);
+// Virtual tokens its plan charges per sequence start: a segment's fixed cost
+// (queries, first tile, merge of its two halves) is about two tiles.
+constexpr int kDecodeF32SegTokens = 64;
+// Pieces per compute unit of an f32 decode.
+inline int decode_f32_blocks_per_cu(int32_t r, int32_t dr) { return decode_f32_mfma_supported(r, dr) ? 1 : 4; }
+qmla_status launch_decode_f32_mfma(const DecodeArgs &a, hipStream_t stream);
 bool decode_mfma_supported(int32_t rows, int32_t r, int32_t dr);
 // Whether a decode with `rows` query rows per sequence over cache `c` has a
 // core (bf16 MFMA shapes, f32 width and row limits); checks no lengths.

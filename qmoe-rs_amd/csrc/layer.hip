@@ -854,7 +854,7 @@ size_t decode_bytes_for(const qmla_layer *L, const qmla_kv_cache *c, int32_t bat
   const bool mfma = c->dtype == QMLA_BF16;
   const int per_cu = mfma && decode_mfma_supported(rows, r, dr)
                          ? decode_mfma_blocks_per_cu(rows, r, dr)
-                         : 4;
+                         : decode_f32_blocks_per_cu(r, dr);
   const int32_t blocks = (int32_t)std::min<int64_t>((int64_t)cus * per_cu, kMaxPlanBlocks);
   return decode_workspace_layout(batch, rows, r, blocks, mfma).total;
 }

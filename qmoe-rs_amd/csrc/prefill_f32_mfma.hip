@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_prefill_f32_mfma(
   // per-lane read offsets inside a chunk
   const uint32_t kread = col * 256 + ((half ^ (col & 15)) << 4);  // piece 2 j + half: ^ 32 j
   const uint32_t vread = half * 1024 + col * 4;                   // + 128 (n ^ half)
-  const uint8_t *my = ring + wave * kRingBytes;
+  uint8_t *my = ring + wave * kRingBytes;
 
   int stage = 0;
   for (int kt = wave; kt < ktiles; kt += kWaves) {
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_prefill_f32_mfma(
       const uint32_t next = lds0 + (stage ^ kChunkBytes);
       if (c + 1 < kChunks) issue(kt, c + 1, next);
       else if (kt + kWaves < ktiles) issue(kt + kWaves, 0, next);
-      const uint8_t *base = my + stage;
+      uint8_t *base = my + stage;
       if (c < (kDn + kDr) / 64) {
         // a sum of its own per 32 dims: short chains round less than one long one
 #pragma unroll
@@ -203,6 +203,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_prefill_f32_mfma(
           }
           m_run = mx;
         }
+        // value rows past kend are zeroed: 0 * V is 0 whatever the re-loaded key holds
+        if (kend - kt * kKeys < kKeys)
+          for (int i = (kend - kt * kKeys) * 16 + lane; i < kKeys * 16; i += 64)
+            reinterpret_cast<floatx4_t *>(base)[i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
 #pragma unroll

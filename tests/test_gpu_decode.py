@@ -301,3 +301,41 @@ def test_decode_bf16_large_batch_lds_plan(qmla_gpu, rows_m):
         assert err < TOL_BF16
         assert np.all(out[empty] == 0) and np.all(np.isneginf(lse[empty]))
         np.testing.assert_allclose(lse[~empty], rlse[~empty], atol=2e-2)
+
+
+@pytest.mark.parametrize("rows_m,q_bf16", [(1, False), (16, True), (17, False), (40, False)])
+def test_decode_f32_mfma_edges(qmla_gpu, rows_m, q_bf16):
+    """f32 cache at the 512 | 64 widths: token tiles that end in either half,
+    row blocks of 16 and their remainders, empty sequences, split counts from
+    one piece to more pieces than tiles.  The oracle sums in f32 as well:
+    2e-5 is some 100 units of 2^-24 on sums of up to 700 terms."""
+    q = qmla_gpu
+    lens = [1, 0, 15, 16, 17, 31, 32, 33, 700, 0, 2]
+    cache, rows, offs = make_cache(q, lens, 512, 64, q.F32, 1500 + rows_m, cap_extra=3)
+    b = len(lens)
+    ql, qr = O.normal((b, rows_m, 512), 1501), O.normal((b, rows_m, 64), 1502)
+    if q_bf16:
+        ql, qr = bf16_to_f32(bf16_bits(ql)), bf16_to_f32(bf16_bits(qr))
+    ref, rlse = O.decode_absorbed(ql, qr, rows, offs, np.asarray(lens, np.int32), 0.06)
+    empty = np.asarray(lens) == 0
+    for splits in (0, 1, 7, 300):
+        out, lse = run(q, cache, ql, qr, 0.06, splits=splits, q_dtype=q.BF16 if q_bf16 else q.F32)
+        assert rel_err(out, ref) < 2e-5
+        assert np.all(out[empty] == 0) and np.all(np.isneginf(lse[empty]))
+        np.testing.assert_allclose(lse[~empty], rlse[~empty], rtol=1e-5, atol=1e-5)
+
+
+def test_decode_f32_mfma_large_batch(qmla_gpu):
+    """More than 64 sequences plan through LDS (bound as above)."""
+    q = qmla_gpu
+    lens = O.uniform_int(150, 77, 0, 200).astype(np.int32)
+    lens[::17] = 0
+    cache, rows, offs = make_cache(q, lens, 512, 64, q.F32, 1600)
+    ql, qr = O.normal((150, 16, 512), 1601), O.normal((150, 16, 64), 1602)
+    ref, rlse = O.decode_absorbed(ql, qr, rows, offs, lens, 0.07)
+    live = lens > 0
+    for splits in (0, 200):
+        out, lse = run(q, cache, ql, qr, 0.07, splits=splits)
+        assert rel_err(out, ref) < 2e-5
+        assert np.all(out[~live] == 0) and np.all(np.isneginf(lse[~live]))
+        np.testing.assert_allclose(lse[live], rlse[live], rtol=1e-5, atol=1e-5)

@@ -244,3 +244,17 @@ def test_prefill_f32_unaligned_tensors(qmla_gpu):
     q.fused_prefill_attn(*[x.ptr + 4 for x in bufs], 0.1, True, dims=dims, dtype=q.F32, out=out.ptr + 4)
     got = out.to_numpy(np.float32, (1 + arrs[4].size,))[1:].reshape(arrs[4].shape)
     assert rel_err(got, q.prefill_numpy(*arrs, 0.1, True)) < 2e-5
+
+
+def test_prefill_f32_infinite_last_value(qmla_gpu):
+    """An infinite value in the last key's column 5 makes that column of the
+    last row infinite (not NaN) and no other, though the last key tile is
+    partial."""
+    arrs = inputs(1, 1, 41, 41, 128, 64, 128, 1, 780)
+    ref = O.fused_prefill_attn(*arrs, 0.1, True)
+    arrs[4][0, 0, 40, 5] = np.inf
+    out, _ = gpu_prefill(qmla_gpu, arrs, 0.1, True)
+    assert np.isposinf(out[0, 0, 40, 5])
+    cols = np.arange(128) != 5
+    assert rel_err(out[..., cols], ref[..., cols]) < 2e-5
+    assert np.isfinite(out[0, 0, :32, 5]).all()
