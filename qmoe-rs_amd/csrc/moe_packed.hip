@@ -27,7 +27,7 @@
 // bytes (one ds_read_b128).
 #include <cmath>
 
-#include "internal.hpp"
+#include "moe_internal.hpp"
 
 namespace qmla {
 namespace {
@@ -826,12 +826,15 @@ __device__ long long block_scan1024(long long v, long long *tmp) {
 }
 
 // Token binning (src/moe.rs:56-82 expert_bins): per-expert counts, bin
-// offsets ({first, count} per expert) and the bin position -> slot list.
+// offsets ({first, count} per expert), the bin position -> slot list and, for
+// the grouped path, the bins' tiles.
 // Order within a bin does not change any result (each pair is computed
 // alone).
 __global__ __launch_bounds__(1024) void k_moe_bin(const int32_t *__restrict__ sel, int npairs,
                                                   int E, int2 *__restrict__ ebin,
-                                                  int32_t *__restrict__ pair_slot) {
+                                                  int32_t *__restrict__ pair_slot,
+                                                  int4 *__restrict__ tiles,
+                                                  int32_t *__restrict__ ntiles) {
   __shared__ int cnt[kMaxExperts];
   __shared__ int cur[kMaxExperts];
   __shared__ long long tmp[16];
@@ -861,6 +864,18 @@ __global__ __launch_bounds__(1024) void k_moe_bin(const int32_t *__restrict__ se
     }
     off += c4[i];
   }
+  if (tiles) {  // the bins' tiles of 32 pairs, in expert order
+    long long nt = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) nt += (c4[i] + 31) / 32;
+    __syncthreads();
+    int at = (int)block_scan1024(nt, tmp);
+    if (threadIdx.x == 1023) *ntiles = at + (int)nt;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      for (int j = 0; j < c4[i]; j += 32)
+        tiles[at++] = int4{4 * (int)threadIdx.x + i, cur[4 * threadIdx.x + i] + j, min(32, c4[i] - j), 0};
+  }
   __syncthreads();
   for (int p = threadIdx.x; p < npairs; p += 1024) {
     const int e = sel[p];
@@ -871,11 +886,48 @@ __global__ __launch_bounds__(1024) void k_moe_bin(const int32_t *__restrict__ se
 }
 
 // out[t] = sum over the token's experts in ascending expert order of
-// y[slot] * weight, starting from zero (src/moe.rs:86, :89, :121-125).
+// y[slot] * weight, starting from zero (src/moe.rs:86, :89, :121-125).  V
+// columns per thread; grid (blocks of a token's columns, tokens), so a token's
+// order is found once per block.
+constexpr int kMaxOrder = 64;  // experts per token ordered in LDS
+
+template <int V>
 __global__ __launch_bounds__(256) void k_moe_combine(const float *__restrict__ y,
                                                      const int32_t *__restrict__ sel,
-                                                     const float *__restrict__ selw, int T,
-                                                     int topk, int H, float *__restrict__ out) {
+                                                     const float *__restrict__ selw, int topk, int H,
+                                                     float *__restrict__ out) {
+  typedef float vec_t __attribute__((ext_vector_type(V)));
+  __shared__ int order[kMaxOrder];
+  __shared__ float weight[kMaxOrder];
+  const int64_t t = blockIdx.y;
+  const int32_t *st = sel + t * topk;
+  const int tid = threadIdx.x;
+  if (tid < topk) {
+    int r = 0;
+    for (int j = 0; j < topk; ++j) r += st[j] < st[tid];
+    order[r] = tid;
+    weight[r] = selw[t * topk + tid];
+  }
+  __syncthreads();
+  const int c = (blockIdx.x * 256 + tid) * V;
+  if (c >= H) return;
+  const float *yt = y + t * topk * H + c;
+  vec_t acc = {};
+#pragma unroll 4
+  for (int r = 0; r < topk; ++r) {
+    const vec_t v = *reinterpret_cast<const vec_t *>(yt + (int64_t)order[r] * H);
+#pragma unroll
+    for (int k = 0; k < V; ++k) acc[k] = __fadd_rn(acc[k], __fmul_rn(v[k], weight[r]));
+  }
+  *reinterpret_cast<vec_t *>(out + t * H + c) = acc;
+}
+
+// The same for more experts per token than kMaxOrder: each thread searches
+// the next one.
+__global__ __launch_bounds__(256) void k_moe_combine_search(const float *__restrict__ y,
+                                                            const int32_t *__restrict__ sel,
+                                                            const float *__restrict__ selw, int T,
+                                                            int topk, int H, float *__restrict__ out) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (int64_t)T * H) return;
   const int t = (int)(idx / H), hh = (int)(idx - (int64_t)t * H);
@@ -987,6 +1039,22 @@ MoeWs moe_ws(const qmla_moe_config &c, int32_t T) {
   w.y = take(sizeof(float) * P * H);
   w.total = o;
   return w;
+}
+
+qmla_status launch_combine(const float *y, const int32_t *sel, const float *selw, int T, int topk,
+                           int H, float *out, hipStream_t s) {
+  const int64_t n = (int64_t)T * H;
+  if (topk > kMaxOrder || T > kMaxTileGrid)
+    hipLaunchKernelGGL(k_moe_combine_search, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, y,
+                       sel, selw, T, topk, H, out);
+  else if ((H & 3) == 0 && aligned16(y) && aligned16(out))
+    hipLaunchKernelGGL(k_moe_combine<4>, dim3((H + 1023) / 1024, T), dim3(256), 0, s, y, sel, selw,
+                       topk, H, out);
+  else
+    hipLaunchKernelGGL(k_moe_combine<1>, dim3((H + 255) / 256, T), dim3(256), 0, s, y, sel, selw,
+                       topk, H, out);
+  QMLA_LAUNCH_CHECK("k_moe_combine");
+  return QMLA_OK;
 }
 
 qmla_status check_moe(const qmla_moe_config *c, int32_t T) {
@@ -1102,6 +1170,23 @@ qmla_status qmla_moe_forward(const qmla_moe_config *cfg, const float *xs, int32_
   // The MFMA GEMV blocks read their expert's bin from the routing table
   // themselves; the per-row fallback walks prebuilt bins.
   const bool block_bins = fast_gu && fast_dn;
+  const bool grouped = block_bins && moe_grouped_supported(c, T) && aligned16(gate_weight) &&
+                       aligned16(gate_scales) && aligned16(up_scales) && aligned16(down_scales);
+  if (grouped) {
+    // hmax's region holds the tile table: 16 bytes per tile and the count
+    int4 *tiles = static_cast<int4 *>(at(w.hmax));
+    int32_t *ntiles = reinterpret_cast<int32_t *>(tiles + moe_grouped_max_tiles(P, c.num_experts));
+    QMLA_TRY(launch_moe_grouped_route(c, xs, T, gate_weight, sel, selw, top_experts, top_weights,
+                                      reinterpret_cast<uint8_t *>(ybuf), s));
+    hipLaunchKernelGGL(k_moe_bin, dim3(1), dim3(1024), 0, s, sel, P, c.num_experts, ebin, slots, tiles,
+                       ntiles);
+    QMLA_LAUNCH_CHECK("k_moe_bin");
+    QMLA_TRY(launch_moe_grouped_experts(
+        MoeGrouped{c, P, gate_packed, up_packed, down_packed, gate_scales, up_scales, down_scales, tiles, ntiles,
+                   slots, hbuf, ybuf},
+        s));
+    return launch_combine(ybuf, sel, selw, T, c.top_k, H, out, s);
+  }
   // Decode-sized calls (the logits fit the blocks' LDS table): only the
   // logits are computed up front, over a wide grid, and the gate/up blocks
   // rank the experts and write the routing table.  Otherwise one block per
@@ -1118,7 +1203,8 @@ qmla_status qmla_moe_forward(const qmla_moe_config *cfg, const float *xs, int32_
     QMLA_LAUNCH_CHECK("k_moe_route");
   }
   if (!block_bins) {
-    hipLaunchKernelGGL(k_moe_bin, dim3(1), dim3(1024), 0, s, sel, P, c.num_experts, ebin, slots);
+    hipLaunchKernelGGL(k_moe_bin, dim3(1), dim3(1024), 0, s, sel, P, c.num_experts, ebin, slots,
+                       (int4 *)nullptr, (int32_t *)nullptr);
     QMLA_LAUNCH_CHECK("k_moe_bin");
   }
   PackedArgs gu{};
@@ -1187,10 +1273,7 @@ qmla_status qmla_moe_forward(const qmla_moe_config *cfg, const float *xs, int32_
   dn.out_max = nullptr;
   QMLA_TRY(launch_packed<1>(dn, (int64_t)c.num_experts * dn.slices, fast_dn, s));
 
-  hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n_out + 255) / 256)), dim3(256), 0, s, ybuf,
-                     sel, selw, T, c.top_k, H, out);
-  QMLA_LAUNCH_CHECK("k_moe_combine");
-  return QMLA_OK;
+  return launch_combine(ybuf, sel, selw, T, c.top_k, H, out, s);
 }
 
 }  // extern "C"

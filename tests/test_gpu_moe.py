@@ -236,3 +236,34 @@ def test_moe_forward_skewed_routing(qmla_gpu, H, I):
     out, idx, _ = moe_layer(qmla_gpu, W).forward(xs, return_routing=True)
     assert (idx[:, 0] == 0).all()
     check_moe(qmla_gpu, W, xs, f"skewed H={H} I={I}")
+
+
+@pytest.mark.parametrize("E,k,H,I,T", [
+    (1, 1, 128, 128, 32), (2, 2, 128, 128, 33), (8, 2, 384, 640, 97), (5, 3, 1408, 2176, 50), (4, 4, 4224, 256, 9),
+    (3, 1, 256, 384, 259)])
+def test_moe_grouped_edges(qmla_gpu, E, k, H, I, T):
+    """At least eight pairs per expert: the grouped path, at tile remainders
+    (32 pairs), row blocks past the last row, four-token routing blocks with a
+    remainder and widths beyond one unit per quantising thread.  Its sums are
+    exact integers, so only x's 2^-23 rounding and f32 products remain: 2e-6."""
+    q = qmla_gpu
+    W = O.random_moe_weights(E, k, H, I, 7000 + H + T)
+    xs = O.normal((T, H), 7100 + T)
+    out, idx, wts = moe_layer(q, W).forward(xs, return_routing=True)
+    ref, ridx, rw = O.moe_forward(W, xs, return_routing=True)
+    np.testing.assert_array_equal(idx, ridx)
+    np.testing.assert_allclose(wts, rw, rtol=1e-4, atol=1e-7)
+    assert rel_err(out, ref) < 2e-6
+
+
+def test_moe_grouped_nonfinite_and_zero_tokens(qmla_gpu):
+    """A NaN token poisons its own row only; a zero token gives zeros."""
+    q = qmla_gpu
+    W = O.random_moe_weights(4, 2, 256, 256, 41)
+    xs = O.normal((70, 256), 42)
+    ref = O.moe_forward(W, xs)
+    xs[2, 5], xs[69] = np.nan, 0.0
+    out = moe_layer(q, W).forward(xs)
+    assert np.isnan(out[2]).all() and np.all(out[69] == 0)
+    keep = [i for i in range(69) if i != 2]
+    assert rel_err(out[keep], ref[keep]) < 2e-6
