@@ -290,13 +290,14 @@ struct SplitGemmArgs {
   int bf16ops;
 };
 bool split_gemm_supported(int N, int K);
+// The reduction of a.ksplit planes of partial sums, bias and epilogue.
+qmla_status launch_sg_reduce(const SplitGemmArgs &a, hipStream_t stream);
 // K slices the split GEMM uses for an M x N x K product (1 when its tiles
 // already fill the device), and the partial-sum bytes they need.
 int split_gemm_slices(int M, int N, int K);
 size_t split_gemm_part_bytes(int M, int N, int K);
 // Rows from which the split GEMM runs its 256 x 256 tiles, and below which
-// the layer keeps its rocBLAS path (few rows stream the weights; the split
-// GEMM's tiles would leave most of the device idle).
+// the layer's prefill runs the f32 rows GEMM (its precision below 128 rows).
 constexpr int kSplitGemmBigRows = 4096;
 constexpr int kSplitGemmMinRows = 128;
 // Scratch for the activation records of an [M][K] product.
@@ -308,6 +309,17 @@ qmla_status launch_split_gemm(const SplitGemmArgs &a, void *pack, hipStream_t st
 // activations, or with hi_only (or a.bf16ops) hi-only records of 1 KB.
 qmla_status launch_split_gemm_packed(const SplitGemmArgs &a, const void *xrec, hipStream_t stream,
                                      bool hi_only = false);
+
+// Projections of few token rows (rows_gemm.hip): the products of SplitGemmArgs
+// (w_frag and bf16ops unused, ksplit chosen by the launch, part set) in f32
+// from the f32 weights w [N][K].  M <= 128; x, w and their rows are 16-byte
+// aligned.
+struct RowsGemmArgs {
+  SplitGemmArgs g;
+  const float *w;
+};
+size_t rows_gemm_part_bytes(int M, int N, int K);
+qmla_status launch_rows_gemm(const RowsGemmArgs &a, hipStream_t stream);
 
 // Cache row writer shared by the cache API and the layer: copies/converts
 // n_seqs x n_new rows (row-major [n_seqs, n_new, row_elems]) into sequences

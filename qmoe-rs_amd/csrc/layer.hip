@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) void k_latent_rows(LatentRowsArgs a) {
 // sequence; the split GEMM's activation records of LayerNorm(c) (kv_b_proj's
 // input, K = r: record (tok / 32, c / 16), lane tok % 32 + 32 ((c / 8) % 2),
 // hi and lo halves, or with rec_lo = 0 (bf16 operands) hi-only records of
-// 1 KB); and rope(k_pe) as the attention's k_rope [b, 1, s, dr]
+// 1 KB; no records with rec null) or the f32 rows a.rows; and rope(k_pe) as the attention's k_rope [b, 1, s, dr]
 // in bf16 or f32.  The sequences start empty (forward_prefill checks it),
 // so positions are the token indices, lens is not read, and the wave of
 // each sequence's token 0 sets its length to s.  The grid covers n rounded
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256) void k_prefill_rows(LatentRowsArgs a, int n, u
   const int RB = rec_lo ? 2048 : 1024;  // bytes per record
   if (tok >= n) {
     // the padding rows of the last 32-row record group: zeros
-    if (tok >= (n + 31) / 32 * 32) return;
+    if (!rec || tok >= (n + 31) / 32 * 32) return;
     for (int c8 = lane; c8 < C8; c8 += 64) {
       uint8_t *rp =
           rec + ((int64_t)(tok >> 5) * KS + (c8 >> 1)) * RB + ((tok & 31) + 32 * (c8 & 1)) * 16;
@@ -390,6 +390,12 @@ __global__ __launch_bounds__(256) void k_prefill_rows(LatentRowsArgs a, int n, u
       *reinterpret_cast<floatx4_t *>(dst + 32 * c8) = floatx4_t{v[0], v[1], v[2], v[3]};
       *reinterpret_cast<floatx4_t *>(dst + 32 * c8 + 16) = floatx4_t{v[4], v[5], v[6], v[7]};
     }
+    if (a.rows) {
+      float *y = a.rows + (int64_t)tok * (r + dr) + 8 * c8;
+      *reinterpret_cast<floatx4_t *>(y) = floatx4_t{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<floatx4_t *>(y + 4) = floatx4_t{v[4], v[5], v[6], v[7]};
+    }
+    if (!rec) continue;
     uint8_t *rp = rec + ((int64_t)(tok >> 5) * KS + (c8 >> 1)) * RB + ((tok & 31) + 32 * (c8 & 1)) * 16;
     *reinterpret_cast<u32x4_t *>(rp) =
         u32x4_t{hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16),
@@ -736,8 +742,9 @@ LayerWs layer_ws(const qmla_layer *L, int32_t batch, int32_t seq, size_t dec_byt
   // cache rows from the GEMM epilogues: it needs neither the f32 q, the
   // rocBLAS split of the activations, the LayerNorm'd rows nor the kv_b
   // output, only the activation records
-  const bool sg = use_split_gemm(L) && n >= (size_t)kSplitGemmMinRows;
-  const bool sg_only = sg && use == WsFor::kPrefill;
+  const bool rg = use_split_gemm(L) && n < (size_t)kSplitGemmMinRows;
+  const bool sg = use_split_gemm(L) && !rg;
+  const bool sg_only = (sg || rg) && use == WsFor::kPrefill;
   w.q = take(sg_only ? 1 : sizeof(float) * n * H * (g.qk_nope + g.qk_rope));
   w.kva = take(sizeof(float) * n * (g.kv_lora_rank + g.qk_rope));
   w.qn = take(sizeof(float) * n * H * g.qk_nope);
@@ -771,7 +778,7 @@ LayerWs layer_ws(const qmla_layer *L, int32_t batch, int32_t seq, size_t dec_byt
   if (use != WsFor::kDecode) {
     off = shared;
     w.rows = take(sg ? 1 : sizeof(float) * n * (g.kv_lora_rank + g.qk_rope));
-    w.kvb = take(sg ? 1 : sizeof(float) * n * H * (g.qk_nope + g.v_dim));
+    w.kvb = take(sg || rg ? 1 : sizeof(float) * n * H * (g.qk_nope + g.v_dim));
     w.k = take(sizeof(float) * n * H * g.qk_nope);
     w.v = take(sizeof(float) * n * H * g.v_dim);
     w.kr = take(sizeof(float) * n * g.qk_rope + 4);
@@ -787,6 +794,9 @@ LayerWs layer_ws(const qmla_layer *L, int32_t batch, int32_t seq, size_t dec_byt
                                    split_gemm_part_bytes((int)n, Nkv, g.kv_lora_rank),
                                    split_gemm_part_bytes((int)n, g.hidden, (int)H * g.v_dim),
                                    (size_t)1})
+                  : rg ? std::max({rows_gemm_part_bytes((int)n, N1, g.hidden),
+                                   rows_gemm_part_bytes((int)n, Nkv, g.kv_lora_rank),
+                                   rows_gemm_part_bytes((int)n, g.hidden, (int)H * g.v_dim)})
                        : 1);
     pre_end = off;
   }
@@ -922,12 +932,16 @@ qmla_status qmla_layer_create(const qmla_layer_config *cfg, const float *wq, con
   qmla_status st = QMLA_OK;
   for (auto &w : ws) {
     if (!w.src) continue;  // optional bias
-    void *p = nullptr;
-    if (hipMalloc(&p, w.n * sizeof(float)) != hipSuccess) {
-      st = fail(QMLA_ERR_OOM, "weight allocation failed");
-      break;
+    // wkva lies right behind wq: one [N][hidden] weight for a product of both
+    void *p = L->wq + ws[0].n;
+    if (w.dst != &L->wkva) {
+      const size_t n = w.n + (w.dst == &L->wq ? ws[2].n : 0);
+      if (hipMalloc(&p, n * sizeof(float)) != hipSuccess) {
+        st = fail(QMLA_ERR_OOM, "weight allocation failed");
+        break;
+      }
+      L->allocs.push_back(p);
     }
-    L->allocs.push_back(p);
     *w.dst = static_cast<float *>(p);
     if (hipMemcpy(p, w.src, w.n * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
       st = fail(QMLA_ERR_HIP, "weight upload failed");
@@ -1233,7 +1247,12 @@ qmla_status qmla_layer_forward_prefill(const qmla_layer *L, const float *xs, int
   // and k_rope are written in bf16 (round to nearest even) into the same
   // regions.  An f32 cache keeps the f32 path throughout.
   const bool bfa = cache->dtype == QMLA_BF16 && prefill_bf16_supported(dn, dr, dv);
-  if (use_split_gemm(L) && n >= kSplitGemmMinRows) {
+  if (use_split_gemm(L)) {
+    // From kSplitGemmMinRows rows the projections run on the split GEMM,
+    // below on the f32 rows GEMM, which keeps the f32 products that few rows
+    // always had (V2-Lite widths, against rocBLAS f32 GEMMs: 16 tokens 79 ->
+    // 50 us, 77 133 -> 73, 127 147 -> 89).
+    const bool few = n < kSplitGemmMinRows;
     // Four launches around the attention, all hand-written:
     //   q_proj | kv_a (q split per head and roped in the epilogue, kv_a rows
     //   raw) -> latent rows (LayerNorm, RoPE, cache write) -> kv_b_proj (k, v
@@ -1266,11 +1285,12 @@ qmla_status qmla_layer_forward_prefill(const qmla_layer *L, const float *xs, int
     qa.inv_freq = L->inv_freq;
     qa.mscale = (float)g.rope_mscale;
     void *pack = ws + w.pack;
-    QMLA_TRY(launch_split_gemm(qa, pack, s));
+    QMLA_TRY(few ? launch_rows_gemm({qa, L->wq}, s)  // wkva lies behind wq
+                 : launch_split_gemm(qa, pack, s));
     // the latent rows: cache rows, kv_b_proj's activation records and k_rope
-    uint8_t *krec = reinterpret_cast<uint8_t *>(ws + w.pack2);
+    uint8_t *krec = few ? nullptr : reinterpret_cast<uint8_t *>(ws + w.pack2);
     {
-      const LatentRowsArgs la = latent_rows_args(L, kva, seq, nullptr, cache);
+      const LatentRowsArgs la = latent_rows_args(L, kva, seq, few ? rows : nullptr, cache);
       const dim3 grid((n + 31) / 32 * 8);  // 4 tokens a block, n rounded up to 32
       // r <= 512 (use_split_gemm): one group of 8 values per lane
       const int rec_lo = L->proj_bf16 ? 0 : 1;
@@ -1291,11 +1311,14 @@ qmla_status qmla_layer_forward_prefill(const qmla_layer *L, const float *xs, int
     ka.epi = kSgEpiKvb;
     ka.out0 = k;
     ka.out1 = v;
-    QMLA_TRY(launch_split_gemm_packed(ka, krec, s));
+    ka.x = rows;
+    ka.ldx = r + dr;
+    QMLA_TRY(few ? launch_rows_gemm({ka, L->wkvb}, s)
+                 : launch_split_gemm_packed(ka, krec, s));
     qmla_prefill_dims pd{batch, H, seq, seq, dn, dr, dv, 1, 0};
     // the bf16 attention can write the context straight as o_proj's
     // activation records (whole 32-token blocks per sequence)
-    const bool ctx_rec = bfa && seq % 32 == 0 && prefill_bf16_records_supported(dn, dr, dv);
+    const bool ctx_rec = !few && bfa && seq % 32 == 0 && prefill_bf16_records_supported(dn, dr, dv);
     if (bfa)
       QMLA_TRY(launch_prefill_bf16(pd, (const uint16_t *)qn, (const uint16_t *)qr,
                                    (const uint16_t *)k, (const uint16_t *)kr, (const uint16_t *)v,
@@ -1315,6 +1338,7 @@ qmla_status qmla_layer_forward_prefill(const qmla_layer *L, const float *xs, int
     oa.epi = kSgEpiFinal;
     oa.y = out;
     oa.ldy = g.hidden;
+    if (few) return launch_rows_gemm({oa, L->wo}, s);
     if (ctx_rec) return launch_split_gemm_packed(oa, pack, s, /*hi_only=*/true);
     return launch_split_gemm(oa, pack, s);
   }

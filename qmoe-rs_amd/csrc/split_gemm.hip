@@ -505,33 +505,50 @@ qmla_status sg_launch(const SplitGemmArgs &a, const uint8_t *xrec, hipStream_t s
   QMLA_REQUIRE(a.ksplit >= 1 && a.ksplit <= 65535 && (a.K / 16 / CF::KSC) % a.ksplit == 0 &&
                    (a.ksplit == 1 || a.part),
                QMLA_ERR_SHAPE, "split GEMM: %d K slices", a.ksplit);
-  const int64_t outs = (int64_t)a.M * (a.N / 4);  // reduce threads
-  QMLA_REQUIRE(outs / 256 + 1 <= 0x7fffffff, QMLA_ERR_SHAPE, "split GEMM reduce grid");
-  auto go = [&](auto kern, auto reduce) -> qmla_status {
+  auto go = [&](auto kern) -> qmla_status {
     QMLA_TRY(ensure_dynamic_lds((const void *)kern, lds));
     kern<<<dim3((unsigned)blocks, (unsigned)a.ksplit), dim3(CF::NWV * 64), lds, s>>>(a, xrec);
     QMLA_LAUNCH_CHECK("k_split_gemm");
-    if (a.ksplit > 1) {
-      reduce<<<dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, s>>>(a);
-      QMLA_LAUNCH_CHECK("k_sg_reduce");
-    }
-    return QMLA_OK;
+    return a.ksplit > 1 ? launch_sg_reduce(a, s) : QMLA_OK;
   };
   switch (a.epi) {
     case kSgEpiQkv:
       if (a.out_bf16)
-        return go(k_split_gemm<CF, XLO, WLO, kSgEpiQkv, uint16_t>, k_sg_reduce<kSgEpiQkv, uint16_t>);
-      return go(k_split_gemm<CF, XLO, WLO, kSgEpiQkv, float>, k_sg_reduce<kSgEpiQkv, float>);
+        return go(k_split_gemm<CF, XLO, WLO, kSgEpiQkv, uint16_t>);
+      return go(k_split_gemm<CF, XLO, WLO, kSgEpiQkv, float>);
     case kSgEpiKvb:
       if (a.out_bf16)
-        return go(k_split_gemm<CF, XLO, WLO, kSgEpiKvb, uint16_t>, k_sg_reduce<kSgEpiKvb, uint16_t>);
-      return go(k_split_gemm<CF, XLO, WLO, kSgEpiKvb, float>, k_sg_reduce<kSgEpiKvb, float>);
+        return go(k_split_gemm<CF, XLO, WLO, kSgEpiKvb, uint16_t>);
+      return go(k_split_gemm<CF, XLO, WLO, kSgEpiKvb, float>);
     default:
-      return go(k_split_gemm<CF, XLO, WLO, kSgEpiFinal, float>, k_sg_reduce<kSgEpiFinal, float>);
+      return go(k_split_gemm<CF, XLO, WLO, kSgEpiFinal, float>);
   }
 }
 
 }  // namespace
+
+qmla_status launch_sg_reduce(const SplitGemmArgs &a, hipStream_t s) {
+  const int64_t outs = (int64_t)a.M * (a.N / 4);
+  QMLA_REQUIRE(outs / 256 + 1 <= 0x7fffffff, QMLA_ERR_SHAPE, "split GEMM reduce grid");
+  const dim3 grid((unsigned)((outs + 255) / 256)), block(256);
+  switch (a.epi) {
+    case kSgEpiQkv:
+      if (a.out_bf16)
+        k_sg_reduce<kSgEpiQkv, uint16_t><<<grid, block, 0, s>>>(a);
+      else
+        k_sg_reduce<kSgEpiQkv, float><<<grid, block, 0, s>>>(a);
+      break;
+    case kSgEpiKvb:
+      if (a.out_bf16)
+        k_sg_reduce<kSgEpiKvb, uint16_t><<<grid, block, 0, s>>>(a);
+      else
+        k_sg_reduce<kSgEpiKvb, float><<<grid, block, 0, s>>>(a);
+      break;
+    default: k_sg_reduce<kSgEpiFinal, float><<<grid, block, 0, s>>>(a);
+  }
+  QMLA_LAUNCH_CHECK("k_sg_reduce");
+  return QMLA_OK;
+}
 
 bool split_gemm_supported(int N, int K) { return N > 0 && N % 4 == 0 && K > 0 && K % 32 == 0; }
 

@@ -186,6 +186,35 @@ def test_prefill_split_gemms_at_small_latent_dims(qmla_gpu, dt, b, s):
     assert list(cache.lengths()) == [s + 2] * b
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("dims", [
+    # hidden, heads, qk_nope, qk_rope, v_dim, kv_lora_rank
+    (160, 4, 48, 16, 32, 64),      # uneven K shares, widths that are no whole 64-output tiles
+    (512, 16, 128, 64, 128, 512),  # V2-Lite head shape (hidden reduced)
+])
+@pytest.mark.parametrize("b,s", [(1, 1), (1, 32), (3, 11), (1, 64), (5, 13), (1, 96), (1, 97), (1, 127)])
+def test_prefill_rows_gemm(qmla_gpu, dt, dims, b, s):
+    """forward_prefill of 1 to 127 rows on the f32 rows GEMM, at the edges of
+    its 32-row blocks, against the oracle's decompressed path, then a decode
+    step.  f32 cache: both sides sum at most 512 products in f32 per output
+    (error about 512^0.5 2^-24 = 1.4e-6 each, four projections deep): 2e-5."""
+    q = qmla_gpu
+    hidden, H, dn, dr, dv, r = dims
+    w = O.MlaWeights.random(hidden, H, dn, dr, dv, r, seed=2300 + s)
+    layer = q.MlaLayer(w)
+    xs = O.normal((b, s, hidden), 2301)
+    cache = q.KVCache([s + 1] * b, r, dr, q.F32 if dt == "f32" else q.BF16)
+    out = layer.forward_prefill(xs, cache)
+    ref, (k, v, kr) = O.mla_forward_prefill(w, xs)
+    tol = 2e-5 if dt == "f32" else 2e-2
+    err = rel_err(out, ref)
+    print(f"rows GEMM prefill {dims} {b}x{s} {dt} rel_err={err:.2e}", flush=True)
+    assert err < tol
+    x1 = O.normal((b, 1, hidden), 2310)
+    ref1, _ = O.mla_forward_with_cache(w, x1, k, v, kr, return_cache=True)
+    assert rel_err(layer.forward_with_cache(x1, cache), ref1) < (TOL if dt == "f32" else 2e-2)
+
+
 def _ragged_cache(q, lens, r, dr, dtype, seed, spare=2):
     """A cache whose sequences hold `lens` random latent rows (N(0,1); bf16
     rounded for a bf16 cache) with `spare` free rows each; returns the cache
@@ -351,8 +380,8 @@ def test_prefill_workspace_is_its_own_and_is_enforced(qmla_gpu):
     print(f"B4 S2048 workspace: prefill {pre >> 20} MiB, either call {both >> 20} MiB")
     assert pre < (1 << 30) and pre * 4 < both
     del big
-    # 80 rows run the rocBLAS projections, 128 rows the hand-written split
-    # GEMMs (whose workspace leaves out the regions only rocBLAS uses)
+    # 80 rows run the f32 rows GEMM, 128 rows the split GEMMs (their workspace
+    # leaves out the regions only rocBLAS uses)
     for dt, (b, s) in [(q.F32, (2, 40)), (q.BF16, (2, 40)), (q.F32, (2, 64)), (q.BF16, (2, 64))]:
         cache = q.KVCache([s] * b, r, dr, dt)
         need = layer.prefill_workspace_bytes(cache, b, s)
