@@ -37,8 +37,10 @@ typedef int i32x16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kTokTile = 10;   // vectors per MFMA tile (3 digit columns each)
 constexpr int kSlab = 4096;    // codes of B staged in LDS at once (128 KB)
-constexpr int kMfmaWaves = 4;  // waves per block; each owns 32 rows
-constexpr int kMfmaThreads = 64 * kMfmaWaves;
+constexpr int kMfmaWaves = 4;  // row waves of a block; each owns 32 rows
+constexpr int kPrepWaves = 4;  // waves that find the block's vectors and prepare the B operand
+constexpr int kPrepThreads = 64 * kPrepWaves;
+constexpr int kMfmaThreads = 64 * (kMfmaWaves + kPrepWaves);
 constexpr int kMaxExperts = 4096;
 constexpr int kSelLds = 2048;  // routing tables up to this many pairs are read into LDS
 constexpr int kMaxK = 1 << 20;
@@ -55,6 +57,7 @@ struct PackedArgs {
   int32_t src_div;          // source vector of slot s = s / src_div
   const int2 *ebin;         // per expert {first bin position, pairs} (grid y = expert x
                             //   slices); null: grid y = tiles of kTokTile over `count` slots
+  int32_t early;            // slice 0 requests weights before its bin is known
   int32_t slices;           // with bins: blocks sharing an expert's bin; block
                             //   (e, s) takes its tiles s, s + slices, ...
   const int32_t *slots;     // bin position -> slot (null: identity)
@@ -93,14 +96,18 @@ __device__ __forceinline__ int block_slice(const PackedArgs &a) {
   return binned(a) ? (int)blockIdx.y % a.slices : 0;
 }
 
+// Index among the preparing threads, which are a block's last waves.
+__device__ __forceinline__ int prep_tid() { return (int)threadIdx.x - 64 * kMfmaWaves; }
+
 // Expert e's bin read from the routing table (the pairs p with sel[p] == e,
 // ascending p): returns its size, and with `out` lists the pairs at bin
 // positions [t0, t0 + n) into out[0..n).  Each thread scans a contiguous run
-// of the table; a block scan of the runs' counts orders them.  Every thread
-// of the block calls it (two barriers); tmp holds kMfmaWaves ints.
+// of the table; a block scan of the runs' counts orders them.  Every
+// preparing thread calls it (two barriers of the block; between them the row
+// waves may add up tmp, kPrepWaves ints, too).
 __device__ int sel_bin(const int32_t *sel, int np, int e, int t0, int n, int *out, int *tmp) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int per = (np + kMfmaThreads - 1) / kMfmaThreads;
+  const int tid = prep_tid(), lane = tid & 63, wave = tid >> 6;
+  const int per = (np + kPrepThreads - 1) / kPrepThreads;
   const int lo = min(np, tid * per), hi = min(np, lo + per);
   int c = 0;
   for (int p = lo; p < hi; ++p) c += sel[p] == e;
@@ -114,7 +121,7 @@ __device__ int sel_bin(const int32_t *sel, int np, int e, int t0, int n, int *ou
   __syncthreads();
   int base = 0, total = 0;
 #pragma unroll
-  for (int w = 0; w < kMfmaWaves; ++w) {
+  for (int w = 0; w < kPrepWaves; ++w) {
     base += w < wave ? tmp[w] : 0;
     total += tmp[w];
   }
@@ -131,18 +138,18 @@ __device__ int sel_bin(const int32_t *sel, int np, int e, int t0, int n, int *ou
 }
 
 constexpr int kRankTokens = 256;  // tokens the GEMV blocks rank themselves (LDS table)
-static_assert(kRankTokens <= kMfmaThreads, "rank_tokens gives every token a thread");
+static_assert(kRankTokens <= kPrepThreads, "rank_tokens gives every token a thread");
 
 // rank[t] = rank of expert e among token t's E logits lg[t][*]: the number of
 // experts before it in (logit descending, index ascending) order, the
 // reference's stable descending sort (src/moe.rs:51-82); NaN ranks as -inf.
 // T <= kRankTokens; pow2 groups of threads share a token and add their
 // counts with LDS atomics into rank[], which the caller zeroed before a
-// barrier.  Every thread of the block calls it (one barrier).
+// barrier.  Every preparing thread calls it (one barrier of the block).
 __device__ void rank_tokens(const float *lg, int T, int E, int e, int *rank) {
-  const int tid = threadIdx.x;
+  const int tid = prep_tid();
   int g = 1;
-  while (g * 2 * T <= kMfmaThreads) g *= 2;
+  while (g * 2 * T <= kPrepThreads) g *= 2;
   const int t = tid / g, part = tid - t * g;
   if (t < T) {
     const float *l = lg + t * E;
@@ -161,8 +168,8 @@ __device__ void rank_tokens(const float *lg, int T, int E, int e, int *rank) {
 // bin is the pairs t * topk + rank[t] of the tokens with rank[t] < topk,
 // ascending (the order sel_bin gives for the table those ranks make).
 __device__ int rank_bin(const int *rank, int T, int topk, int t0, int n, int *out, int *tmp) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int per = (T + kMfmaThreads - 1) / kMfmaThreads;
+  const int tid = prep_tid(), lane = tid & 63, wave = tid >> 6;
+  const int per = (T + kPrepThreads - 1) / kPrepThreads;
   const int lo = min(T, tid * per), hi = min(T, lo + per);
   int c = 0;
   for (int t = lo; t < hi; ++t) c += rank[t] < topk;
@@ -176,7 +183,7 @@ __device__ int rank_bin(const int *rank, int T, int topk, int t0, int n, int *ou
   __syncthreads();
   int base = 0, total = 0;
 #pragma unroll
-  for (int w = 0; w < kMfmaWaves; ++w) {
+  for (int w = 0; w < kPrepWaves; ++w) {
     base += w < wave ? tmp[w] : 0;
     total += tmp[w];
   }
@@ -203,12 +210,6 @@ __device__ __forceinline__ void block_range(const PackedArgs &a, int &first, int
   }
 }
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt out of range");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
-}
-
 __device__ __forceinline__ u32x4_t gload16(const uint8_t *p) {
   return *reinterpret_cast<const u32x4_t *>(p);
 }
@@ -222,18 +223,25 @@ constexpr int kBadExp = 0x7fffffff;  // exponent marking a vector with inf/NaN
 
 // Expert GEMV over one tile of vectors.  NMAT = 1: out = dot * scale.
 // NMAT = 2 (gate, up): out = swish(dot_0 * s_0) * (dot_1 * s_1)
-// (src/moe.rs:102-115).  Block: 4 waves x 32 rows; grid (row blocks,
-// experts) with each block walking its expert's tiles, or (row blocks,
-// tiles) without bins.
-// The block turns its <= 10 f32 vectors into digit planes itself: pass 1
-// finds each vector's largest magnitude (its exponent e) unless the producer
-// handed it over (src_max), pass 2 writes the digits of each slab of K into
-// LDS in the lane order of the B operand and sums q per vector.
+// (src/moe.rs:102-115).  Block: 4 row waves x 32 rows and 4 preparing waves;
+// grid (row blocks, experts) with each block walking its expert's tiles, or
+// (row blocks, tiles) without bins.
+// The preparing waves find the block's <= 10 f32 vectors and turn them into
+// digit planes: pass 1 finds each vector's largest magnitude (its exponent e)
+// unless the producer handed it over (src_max), pass 2 writes the digits of
+// each slab of K into LDS in the lane order of the B operand and sums q per
+// vector.  Meanwhile the row waves' weight loads are in flight.  The roles are
+// apart because a wave's loads return in order: when one wave did both, its
+// routing table and vectors waited behind the weights (9 of the gate/up
+// block's 24 us).  1 token over 32 experts, 2048 x 1408: 34.3 -> 26.9 us; 8
+// tokens 41.2 -> 38.2; 16 tokens 44.2 -> 42.2, bound by the digit passes of
+// the fuller bins and the row waves' MFMAs on CUs with two blocks.  128
+// registers, so that two blocks fit a CU.  The two roles meet at the block's
+// barriers, numbered alike on both sides.
 // NG > 0: K = 128 NG in one slab with a compile-time ring of weight
-// groups, the first ones requested at entry so their HBM latency overlaps
-// the quantisation.  NG = 0: any K % 128 == 0, a ring of D groups in flight.
+// groups.  NG = 0: any K % 128 == 0, a ring of D groups in flight.
 template <int NMAT, int NG>
-__global__ __launch_bounds__(kMfmaThreads) void k_packed_mfma(PackedArgs a) {
+__global__ __launch_bounds__(kMfmaThreads, 4) void k_packed_mfma(PackedArgs a) {
   extern __shared__ __attribute__((aligned(16))) int8_t lds_b[];  // [chunk][h][32][16]
   __shared__ int64_t voff[kTokTile];
   __shared__ int vslot[kTokTile];
@@ -242,366 +250,395 @@ __global__ __launch_bounds__(kMfmaThreads) void k_packed_mfma(PackedArgs a) {
   __shared__ unsigned long long vsum[kTokTile];
   __shared__ unsigned bmax[kTokTile];
   __shared__ int sel_list[kTokTile];
-  __shared__ int sel_tmp[kMfmaWaves];
+  __shared__ int sel_tmp[kPrepWaves];
   __shared__ int32_t sel_lds[kSelLds];
   __shared__ int rank_lds[kRankTokens];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int expert = block_expert(a), slice = block_slice(a);
+  const int tt0 = slice * kTokTile;
+  // without bins the grid position is the block's only tile (count <= kTokTile)
+  const int tstep = binned(a) ? a.slices * kTokTile : kTokTile;
+  const bool table = a.sel && a.npairs <= kSelLds;  // read once, into LDS
+
+  if (wave >= kMfmaWaves) {
+    // ---- preparing waves
+    const int tid = prep_tid();
+    int first = 0, count;
+    const int32_t *bins = a.sel;
+    const float *lg = reinterpret_cast<const float *>(sel_lds);
+    const int ntok_r = a.logits ? a.npairs / a.topk : 0;
+    if (a.logits) {  // (always in LDS: the host takes this path only when they fit)
+      for (int i = tid; i < ntok_r * a.n_experts; i += kPrepThreads)
+        sel_lds[i] = __float_as_int(a.logits[i]);
+      for (int t = tid; t < ntok_r; t += kPrepThreads) rank_lds[t] = 0;
+      __syncthreads();  // (1)
+      rank_tokens(lg, ntok_r, a.n_experts, expert, rank_lds);  // (2)
+      count = rank_bin(rank_lds, ntok_r, a.topk, tt0, kTokTile, sel_list, sel_tmp);  // (3)
+    } else if (a.sel) {
+      if (table) {
+        for (int p = tid; p < a.npairs; p += kPrepThreads) sel_lds[p] = a.sel[p];
+        __syncthreads();  // (1)
+        bins = sel_lds;
+      }
+      count = sel_bin(bins, a.npairs, expert, tt0, kTokTile, sel_list, sel_tmp);  // (3)
+    } else {
+      block_range(a, first, count);
+    }
+    for (int tt = tt0; tt < count; tt += tstep) {
+      const int ntok = min(kTokTile, count - tt);
+      if (tt != tt0) {  // (the first tile's vectors came with the count)
+        __syncthreads();  // (4)
+        if (a.logits)
+          rank_bin(rank_lds, ntok_r, a.topk, tt, ntok, sel_list, sel_tmp);  // (5)
+        else if (a.sel)
+          sel_bin(bins, a.npairs, expert, tt, ntok, sel_list, sel_tmp);  // (5)
+      }
+      // 16 lanes per vector: its slot, source and, where the producer left
+      // partial maxima, their maximum
+      if (tid < 16 * kTokTile) {
+        const int t = tid >> 4, j = tid & 15;
+        unsigned m = 0;
+        if (t < ntok) {
+          const int pos = first + tt + t;
+          const int slot = a.sel || a.logits ? sel_list[t] : a.slots ? a.slots[pos] : pos;
+          const int src = slot / a.src_div;
+          if (j == 0) {
+            vslot[t] = slot;
+            voff[t] = (int64_t)src * a.ld_x;
+          }
+          if (a.src_max)
+            for (int q = j; q < a.src_max_parts; q += 16)
+              m = max(m, a.src_max[(int64_t)src * a.src_max_parts + q]);
+        }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+        if (j == 0) {
+          vmax[t] = m;
+          vsum[t] = 0;
+          bmax[t] = 0;
+        }
+      }
+      __syncthreads();  // (6)
+
+      const int K4 = a.K >> 2;
+      if (!a.src_max) {
+        // Pass 1: largest |x| of each vector (as f32 bits; inf/NaN compare above).
+        const int items = ntok * K4;
+        constexpr int U = 8;
+        unsigned run = 0;
+        int cur = -1;
+        for (int base = 0; base < items; base += kPrepThreads * U) {
+          u32x4_t v[U];
+          int vt[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int i = min(base + tid + kPrepThreads * u, items - 1);
+            const int tu = i / K4;
+            v[u] = *reinterpret_cast<const u32x4_t *>(a.x + voff[tu] + 4 * (i - tu * K4));
+            vt[u] = base + tid + kPrepThreads * u < items ? tu : -1;
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            if (vt[u] < 0) continue;
+            if (vt[u] != cur) {
+              if (cur >= 0) atomicMax(&vmax[cur], run);
+              cur = vt[u];
+              run = 0;
+            }
+            const u32x4_t m = v[u] & 0x7fffffffu;
+            run = max(run, max(max(m[0], m[1]), max(m[2], m[3])));
+          }
+        }
+        if (cur >= 0) atomicMax(&vmax[cur], run);
+        __syncthreads();  // (7)
+      }
+      if (tid < ntok) {
+        const unsigned mb = vmax[tid] & 0x7fffffffu;
+        int e = 0;
+        if (mb >= 0x7f800000u) {
+          e = kBadExp;
+        } else if (mb != 0) {
+          int ex;
+          frexpf(__uint_as_float(mb), &ex);  // max |x| < 2^ex
+          e = 22 - ex;                       // max |q| <= 2^22
+        }
+        vexp[tid] = e;
+      }
+
+      for (int k0 = 0; k0 < a.K; k0 += kSlab) {
+        const int nch = min(kSlab, a.K - k0) >> 5;
+        __syncthreads();  // (8)
+        // Pass 2: digit planes of the slab.  Item (t, half, chunk) covers 16
+        // consecutive k of vector t and fills columns 3t .. 3t+2.
+        const int items = ntok * 2 * nch;
+        unsigned long long qs = 0;
+        int cur = -1;
+        constexpr int U2 = 2;  // items whose loads are issued together
+        for (int i0 = tid; i0 < items; i0 += kPrepThreads * U2) {
+          floatx4_t f[U2][4];
+#pragma unroll
+          for (int u = 0; u < U2; ++u) {
+            const int i = min(i0 + kPrepThreads * u, items - 1);
+            const int t = i % ntok, r = i / ntok;
+            const int cg = (k0 >> 5) + (r >> 1);
+            const float *src = a.x + voff[t] + 128 * (cg >> 2) + 64 * (r & 1) + 16 * (cg & 3);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) f[u][j] = *reinterpret_cast<const floatx4_t *>(src + 4 * j);
+          }
+#pragma unroll
+          for (int u = 0; u < U2; ++u) {
+            const int i = i0 + kPrepThreads * u;
+            if (i >= items) break;
+            const int t = i % ntok, r = i / ntok;
+            const int h2 = r & 1, c = r >> 1;
+            const int e = vexp[t];
+            uint32_t w0[4] = {0, 0, 0, 0}, w1[4] = {0, 0, 0, 0}, w2[4] = {0, 0, 0, 0};
+            long long sq = 0;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {  // j = 4 b + v -> byte b of word v
+              const int q = e == kBadExp ? 0 : (int)rintf(ldexpf(f[u][j >> 2][j & 3], e));
+              const int d0 = ((q + 128) & 255) - 128;
+              const int q1 = (q - d0) >> 8;
+              const int d1 = ((q1 + 128) & 255) - 128;
+              const int d2 = (q1 - d1) >> 8;
+              const int v = j & 3, sh = 8 * (j >> 2);
+              w0[v] |= (uint32_t)(d0 & 255) << sh;
+              w1[v] |= (uint32_t)(d1 & 255) << sh;
+              w2[v] |= (uint32_t)(d2 & 255) << sh;
+              sq += q;
+            }
+            i32x4_t *dst = reinterpret_cast<i32x4_t *>(lds_b + (((c * 2 + h2) * 32 + 3 * t) << 4));
+            dst[0] = i32x4_t{(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3]};
+            dst[1] = i32x4_t{(int)w1[0], (int)w1[1], (int)w1[2], (int)w1[3]};
+            dst[2] = i32x4_t{(int)w2[0], (int)w2[1], (int)w2[2], (int)w2[3]};
+            if (t != cur) {
+              if (cur >= 0) atomicAdd(&vsum[cur], qs);
+              cur = t;
+              qs = 0;
+            }
+            qs += (unsigned long long)sq;
+          }
+        }
+        if (cur >= 0) atomicAdd(&vsum[cur], qs);
+        __syncthreads();  // (9)
+      }
+      __syncthreads();  // (10)
+      if (a.out_max) {  // this block's partial maximum per vector, no global atomics
+        __syncthreads();  // (11)
+        if (tid < ntok) a.out_max[(int64_t)vslot[tid] * gridDim.x + blockIdx.x] = bmax[tid];
+      }
+    }
+    if (a.sel_out && slice == 0) {
+      // This expert's part of the routing table, for the launches after this
+      // one: (expert, weight) at pair t * topk + rank.  The weight is the
+      // softmax over all experts' logits (src/moe.rs:51-82), one wave per
+      // token with k_moe_route's lane order and reductions; the expert's row
+      // blocks share the tokens (token t: row block t % gridDim.x).
+      const int E = a.n_experts;
+      for (int t = blockIdx.x + (int)gridDim.x * (wave - kMfmaWaves); t < ntok_r;
+           t += (int)gridDim.x * kPrepWaves) {
+        if (rank_lds[t] >= a.topk) continue;
+        const float *l = lg + t * E;
+        float mx = -INFINITY;
+        for (int j = lane; j < E; j += 64) mx = fmaxf(mx, l[j]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+        float se = 0.f;
+        for (int j = lane; j < E; j += 64) se += expf(l[j] - mx);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o);
+        if (lane == 0) {
+          const float w = expf(l[expert] - mx) / se;
+          const int o = t * a.topk + rank_lds[t];
+          a.sel_out[o] = expert;
+          a.selw_out[o] = w;
+          if (a.user_idx) a.user_idx[o] = expert;
+          if (a.user_w) a.user_w[o] = w;
+        }
+      }
+    }
+    return;
+  }
+
+  // ---- row waves
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
   const int n = lane & 31, h = lane >> 5;
   const int m0 = (blockIdx.x * kMfmaWaves + wave) * 32;
   const bool wave_ok = m0 < a.M;
-  const bool row_ok = m0 + n < a.M;
+  const int row = m0 + n;
+  const bool row_ok = row < a.M;
   const int bpr = a.K >> 2;
-  const int expert = block_expert(a), slice = block_slice(a);
   const uint8_t *wp[NMAT];
 #pragma unroll
   for (int i = 0; i < NMAT; ++i)
-    wp[i] = a.w[i] + expert * a.w_stride + (int64_t)(row_ok ? m0 + n : 0) * bpr + 16 * h;
+    wp[i] = a.w[i] + expert * a.w_stride + (int64_t)(row_ok ? row : 0) * bpr + 16 * h;
 
   // Loads are branch-free (rows past M read row 0, ring slots past the slab
   // re-read its last group; neither result is used) so that the compiler
-  // keeps them in flight instead of waiting behind each branch.  The first
-  // groups are requested before the block knows its tokens: the expert is
-  // the grid position, so the weight stream starts while the bins are read.
+  // keeps them in flight instead of waiting behind each branch.
   constexpr int D = 4;
-  constexpr int PD = NMAT == 1 ? 8 : 6;  // groups in flight, fixed group count
+  constexpr int PD = NMAT == 1 ? 11 : 8;  // groups in flight, fixed group count
   constexpr int NR = NG > 0 ? (NG < PD ? NG : PD) : D;
   u32x4_t ring[NR][NMAT];
   const int ng0 = min(kSlab, a.K) >> 7;
-  // Slice 0 requests its first weight groups before it reads its bin; the
-  // other slices of an expert (which have work only for bins of more than
-  // one tile) request theirs once they know they have a tile.
-  if (slice == 0) {
+  auto request = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int d = 0; d < NR; ++d)
 #pragma unroll
       for (int i = 0; i < NMAT; ++i)
         ring[d][i] = gload16(wp[i] + (NG > 0 ? d : min(d, ng0 - 1)) * 32);
-  }
+  };
+  const int rowc = row_ok ? row : 0;
+  const float sc0 = a.scale[0][expert * a.s_stride + rowc];
+  const float sc1 = a.scale[NMAT - 1][expert * a.s_stride + rowc];
+  // Slice 0 requests its first weight groups before its bin is known when
+  // most experts have one (a.early); the other slices of an expert (which have
+  // work only for bins of more than one tile) once they know they have a tile.
+  const bool early = slice == 0 && a.early;
+  if (early) request();
 
-  int first = 0, count;
-  // the routing table, read once (into LDS when it fits); or the logits
-  // (always in LDS: the host takes this path only when they fit)
-  const int32_t *bins = a.sel;
-  const float *lg = reinterpret_cast<const float *>(sel_lds);
-  const int ntok_r = a.logits ? a.npairs / a.topk : 0;
-  if (a.logits) {
-    for (int i = tid; i < ntok_r * a.n_experts; i += kMfmaThreads)
-      sel_lds[i] = __float_as_int(a.logits[i]);
-    for (int t = tid; t < ntok_r; t += kMfmaThreads) rank_lds[t] = 0;
-    __syncthreads();
-  } else if (a.sel && a.npairs <= kSelLds) {
-    for (int p = tid; p < a.npairs; p += kMfmaThreads) sel_lds[p] = a.sel[p];
-    __syncthreads();
-    bins = sel_lds;
-  }
-  if (a.logits) {
-    rank_tokens(lg, ntok_r, a.n_experts, expert, rank_lds);
-    count = rank_bin(rank_lds, ntok_r, a.topk, 0, 0, nullptr, sel_tmp);
-  } else if (a.sel) {
-    count = sel_bin(bins, a.npairs, expert, 0, 0, nullptr, sel_tmp);
+  // the preparing waves' barriers; the bin's size from their counts
+  int count;
+  if (a.logits || a.sel) {
+    if (a.logits || table) __syncthreads();  // (1)
+    if (a.logits) __syncthreads();           // (2)
+    __syncthreads();                         // (3)
+    count = 0;
+#pragma unroll
+    for (int w = 0; w < kPrepWaves; ++w) count += sel_tmp[w];
+    __syncthreads();  // (3)
   } else {
+    int first;
     block_range(a, first, count);
   }
-  if (a.sel_out && slice == 0) {
-    // This expert's part of the routing table, for the launches after this
-    // one: (expert, weight) at pair t * topk + rank.  The weight is the
-    // softmax over all experts' logits (src/moe.rs:51-82), one wave per
-    // token with k_moe_route's lane order and reductions; the expert's row
-    // blocks share the tokens (token t: row block t % gridDim.x).
-    const int E = a.n_experts, lane = tid & 63, wave = tid >> 6;
-    for (int t = blockIdx.x + (int)gridDim.x * wave; t < ntok_r;
-         t += (int)gridDim.x * kMfmaWaves) {
-      if (rank_lds[t] >= a.topk) continue;
-      const float *l = lg + t * E;
-      float mx = -INFINITY;
-      for (int j = lane; j < E; j += 64) mx = fmaxf(mx, l[j]);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-      float se = 0.f;
-      for (int j = lane; j < E; j += 64) se += expf(l[j] - mx);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o);
-      if (lane == 0) {
-        const float w = expf(l[expert] - mx) / se;
-        const int o = t * a.topk + rank_lds[t];
-        a.sel_out[o] = expert;
-        a.selw_out[o] = w;
-        if (a.user_idx) a.user_idx[o] = expert;
-        if (a.user_w) a.user_w[o] = w;
-      }
-    }
-  }
-  const int tt0 = slice * kTokTile;
-  if (count <= tt0) {  // no tile for this block: drain the requested groups
-    wait_vm<0>();
-    return;
-  }
-  // without bins the grid position is the block's only tile (count <= kTokTile)
-  const int tstep = binned(a) ? a.slices * kTokTile : kTokTile;
   for (int tt = tt0; tt < count; tt += tstep) {
-  const TileInfo ti{expert, first + tt, min(kTokTile, count - tt)};
-  if (tt != tt0 || slice != 0) {
-    // a later tile of this block: the LDS of the last one is free once every
-    // wave is past its epilogue; its weights come again (from L2)
-    if (tt != tt0) __syncthreads();
-#pragma unroll
-    for (int d = 0; d < NR; ++d)
-#pragma unroll
-      for (int i = 0; i < NMAT; ++i)
-        ring[d][i] = gload16(wp[i] + (NG > 0 ? d : min(d, ng0 - 1)) * 32);
-  }
-
-  if (a.logits)
-    rank_bin(rank_lds, ntok_r, a.topk, tt, ti.ntok, sel_list, sel_tmp);
-  else if (a.sel)
-    sel_bin(bins, a.npairs, expert, tt, ti.ntok, sel_list, sel_tmp);
-  if (tid < kTokTile) {
-    vmax[tid] = 0;
-    vsum[tid] = 0;
-    if (tid < ti.ntok) {
-      const int pos = ti.start + tid;
-      const int slot = a.sel || a.logits ? sel_list[tid] : a.slots ? a.slots[pos] : pos;
-      const int src = slot / a.src_div;
-      vslot[tid] = slot;
-      voff[tid] = (int64_t)src * a.ld_x;
-      if (a.src_max) {
-        unsigned m = 0;
-        for (int j = 0; j < a.src_max_parts; ++j)
-          m = max(m, a.src_max[(int64_t)src * a.src_max_parts + j]);
-        vmax[tid] = m;
+    const int ntok = min(kTokTile, count - tt);
+    // a later tile of this block: its weights come again (from L2), and the
+    // LDS of the last one is free once every wave is past its epilogue
+    if (tt != tt0 || !early) request();
+    if (tt != tt0) {
+      __syncthreads();  // (4)
+      if (a.logits || a.sel) {
+        __syncthreads();  // (5)
+        __syncthreads();
       }
     }
-    bmax[tid] = 0;
-  }
-  __syncthreads();
+    __syncthreads();                  // (6)
+    if (!a.src_max) __syncthreads();  // (7)
 
-  const int K4 = a.K >> 2;
-  if (!a.src_max) {
-    // Pass 1: largest |x| of each vector (as f32 bits; inf/NaN compare above).
-    const int items = ti.ntok * K4;
-    constexpr int U = 8;
-    unsigned run = 0;
-    int cur = -1;
-    for (int base = 0; base < items; base += kMfmaThreads * U) {
-      u32x4_t v[U];
-      int tt[U];
+    i32x16_t acc[NMAT];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = min(base + tid + kMfmaThreads * u, items - 1);
-        const int tu = i / K4;
-        v[u] = *reinterpret_cast<const u32x4_t *>(a.x + voff[tu] + 4 * (i - tu * K4));
-        tt[u] = base + tid + kMfmaThreads * u < items ? tu : -1;
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (tt[u] < 0) continue;
-        if (tt[u] != cur) {
-          if (cur >= 0) atomicMax(&vmax[cur], run);
-          cur = tt[u];
-          run = 0;
-        }
-        const u32x4_t m = v[u] & 0x7fffffffu;
-        run = max(run, max(max(m[0], m[1]), max(m[2], m[3])));
-      }
-    }
-    if (cur >= 0) atomicMax(&vmax[cur], run);
-    __syncthreads();
-  }
-  if (tid < ti.ntok) {
-    const unsigned mb = vmax[tid] & 0x7fffffffu;
-    int e = 0;
-    if (mb >= 0x7f800000u) {
-      e = kBadExp;
-    } else if (mb != 0) {
-      int ex;
-      frexpf(__uint_as_float(mb), &ex);  // max |x| < 2^ex
-      e = 22 - ex;                       // max |q| <= 2^22
-    }
-    vexp[tid] = e;
-  }
-
-  i32x16_t acc[NMAT];
-#pragma unroll
-  for (int i = 0; i < NMAT; ++i) acc[i] = i32x16_t{};
-
-  for (int k0 = 0; k0 < a.K; k0 += kSlab) {
-    const int ks = min(kSlab, a.K - k0);
-    const int nch = ks >> 5;
-    __syncthreads();
-    // Pass 2: digit planes of the slab.  Item (t, half, chunk) covers 16
-    // consecutive k of vector t and fills columns 3t .. 3t+2.
-    {
-      const int items = ti.ntok * 2 * nch;
-      unsigned long long qs = 0;
-      int cur = -1;
-      constexpr int U2 = 2;  // items whose loads are issued together
-      for (int i0 = tid; i0 < items; i0 += kMfmaThreads * U2) {
-        floatx4_t f[U2][4];
-#pragma unroll
-        for (int u = 0; u < U2; ++u) {
-          const int i = min(i0 + kMfmaThreads * u, items - 1);
-          const int t = i % ti.ntok, r = i / ti.ntok;
-          const int cg = (k0 >> 5) + (r >> 1);
-          const float *src = a.x + voff[t] + 128 * (cg >> 2) + 64 * (r & 1) + 16 * (cg & 3);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) f[u][j] = *reinterpret_cast<const floatx4_t *>(src + 4 * j);
-        }
-#pragma unroll
-        for (int u = 0; u < U2; ++u) {
-          const int i = i0 + kMfmaThreads * u;
-          if (i >= items) break;
-          const int t = i % ti.ntok, r = i / ti.ntok;
-          const int h2 = r & 1, c = r >> 1;
-          const int e = vexp[t];
-          uint32_t w0[4] = {0, 0, 0, 0}, w1[4] = {0, 0, 0, 0}, w2[4] = {0, 0, 0, 0};
-          long long sq = 0;
-#pragma unroll
-          for (int j = 0; j < 16; ++j) {  // j = 4 b + v -> byte b of word v
-            const int q = e == kBadExp ? 0 : (int)rintf(ldexpf(f[u][j >> 2][j & 3], e));
-            const int d0 = ((q + 128) & 255) - 128;
-            const int q1 = (q - d0) >> 8;
-            const int d1 = ((q1 + 128) & 255) - 128;
-            const int d2 = (q1 - d1) >> 8;
-            const int v = j & 3, sh = 8 * (j >> 2);
-            w0[v] |= (uint32_t)(d0 & 255) << sh;
-            w1[v] |= (uint32_t)(d1 & 255) << sh;
-            w2[v] |= (uint32_t)(d2 & 255) << sh;
-            sq += q;
-          }
-          i32x4_t *dst = reinterpret_cast<i32x4_t *>(lds_b + (((c * 2 + h2) * 32 + 3 * t) << 4));
-          dst[0] = i32x4_t{(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3]};
-          dst[1] = i32x4_t{(int)w1[0], (int)w1[1], (int)w1[2], (int)w1[3]};
-          dst[2] = i32x4_t{(int)w2[0], (int)w2[1], (int)w2[2], (int)w2[3]};
-          if (t != cur) {
-            if (cur >= 0) atomicAdd(&vsum[cur], qs);
-            cur = t;
-            qs = 0;
-          }
-          qs += (unsigned long long)sq;
-        }
-      }
-      if (cur >= 0) atomicAdd(&vsum[cur], qs);
+    for (int i = 0; i < NMAT; ++i) acc[i] = i32x16_t{};
+    for (int k0 = 0; k0 < (NG > 0 ? 1 : a.K); k0 += kSlab) {  // NG > 0: one slab
+      const int ks = NG > 0 ? 128 * NG : min(kSlab, a.K - k0);
+      const int nch = ks >> 5;
+      __syncthreads();  // (8)
       // columns of absent vectors and the two spare columns
-      const int spare = 32 - 3 * ti.ntok;
-      for (int i = tid; i < spare * 2 * nch; i += kMfmaThreads) {
-        const int col = 3 * ti.ntok + i % spare, r = i / spare;
+      const int spare = 32 - 3 * ntok;
+      for (int i = tid; i < spare * 2 * nch; i += 64 * kMfmaWaves) {
+        const int col = 3 * ntok + i % spare, r = i / spare;
         *reinterpret_cast<i32x4_t *>(lds_b + ((r * 32 + col) << 4)) = i32x4_t{0, 0, 0, 0};
       }
-    }
-    __syncthreads();
-    // Nothing but weight loads is in flight from here on: without this
-    // drain the compiler keeps waits at the loop head for loads of the
-    // passes above, which would also hold the weight ring.  The weights
-    // were requested before pass 1.
-    wait_vm<0>();
-    if (!wave_ok) continue;
-    if constexpr (NG > 0) {
+      __syncthreads();  // (9)
+      if (!wave_ok) continue;
+      if constexpr (NG > 0) {
 #pragma unroll
-      for (int g = 0; g < NG; ++g) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const i32x4_t b = *reinterpret_cast<const i32x4_t *>(
-              lds_b + ((((g * 4 + c) * 2 + h) * 32 + n) << 4));
-#pragma unroll
-          for (int i = 0; i < NMAT; ++i)
-            acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(decode_codes(ring[g % NR][i][c]), b,
-                                                           acc[i], 0, 0, 0);
-        }
-        if (g + NR < NG) {  // compile-time: refill the slot with group g + NR
-#pragma unroll
-          for (int i = 0; i < NMAT; ++i) ring[g % NR][i] = gload16(wp[i] + (g + NR) * 32);
-        }
-        // pin the refill here: the scheduler would otherwise sink it next
-        // to its use and leave one group in flight
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-      const int ng = ks >> 7;
-      const int gk0 = k0 >> 7;
-      if (k0 > 0) {
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-#pragma unroll
-          for (int i = 0; i < NMAT; ++i)
-            ring[d][i] = gload16(wp[i] + (gk0 + min(d, ng - 1)) * 32);
-      }
-      // Branch-free body (the group count is padded to a multiple of D;
-      // padding groups multiply zero codes), so that the compiler's waits
-      // stay per group instead of collapsing at each branch.
-      for (int g0 = 0; g0 < ng; g0 += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-          const int g = g0 + d;
-          const bool live = g < ng;
-          const int gl = min(g, ng - 1);
+        for (int g = 0; g < NG; ++g) {
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             const i32x4_t b = *reinterpret_cast<const i32x4_t *>(
-                lds_b + ((((gl * 4 + c) * 2 + h) * 32 + n) << 4));
+                lds_b + ((((g * 4 + c) * 2 + h) * 32 + n) << 4));
 #pragma unroll
             for (int i = 0; i < NMAT; ++i)
-              acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                  decode_codes(live ? ring[d][i][c] : 0u), b, acc[i], 0, 0, 0);
+              acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(decode_codes(ring[g % NR][i][c]), b,
+                                                             acc[i], 0, 0, 0);
           }
-          // the slot is free once its codes are decoded: refill it in place
+          if (g + NR < NG) {  // compile-time: refill the slot with group g + NR
 #pragma unroll
-          for (int i = 0; i < NMAT; ++i)
-            ring[d][i] = gload16(wp[i] + (gk0 + min(g + D, ng - 1)) * 32);
+            for (int i = 0; i < NMAT; ++i) ring[g % NR][i] = gload16(wp[i] + (g + NR) * 32);
+          }
+          // pin the refill here: the scheduler would otherwise sink it next
+          // to its use and leave one group in flight
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        const int ng = ks >> 7;
+        const int gk0 = k0 >> 7;
+        if (k0 > 0) {
+#pragma unroll
+          for (int d = 0; d < D; ++d)
+#pragma unroll
+            for (int i = 0; i < NMAT; ++i)
+              ring[d][i] = gload16(wp[i] + (gk0 + min(d, ng - 1)) * 32);
+        }
+        // Branch-free body (the group count is padded to a multiple of D;
+        // padding groups multiply zero codes), so that the compiler's waits
+        // stay per group instead of collapsing at each branch.
+        for (int g0 = 0; g0 < ng; g0 += D) {
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            const int g = g0 + d;
+            const bool live = g < ng;
+            const int gl = min(g, ng - 1);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const i32x4_t b = *reinterpret_cast<const i32x4_t *>(
+                  lds_b + ((((gl * 4 + c) * 2 + h) * 32 + n) << 4));
+#pragma unroll
+              for (int i = 0; i < NMAT; ++i)
+                acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                    decode_codes(live ? ring[d][i][c] : 0u), b, acc[i], 0, 0, 0);
+            }
+            // the slot is free once its codes are decoded: refill it in place
+#pragma unroll
+            for (int i = 0; i < NMAT; ++i)
+              ring[d][i] = gload16(wp[i] + (gk0 + min(g + D, ng - 1)) * 32);
+          }
         }
       }
     }
-  }
-  // Epilogue.  The accumulators go through LDS (the B area, free once
-  // every wave is past its MFMAs) so that each lane finishes whole outputs:
-  // row rl = lane % 32 of the wave's 32, vectors lane / 32, + 2, ...  The
-  // three digit columns are combined once per output and each vector's 32
-  // rows leave as one 128-byte store.  Idle waves (rows past M) stay to the
-  // end for the block barriers.
-  __syncthreads();
-  int *accs = reinterpret_cast<int *>(lds_b) + wave * (NMAT * 16 * 64);
-  if (wave_ok) {
+    // Epilogue.  The accumulators go through LDS (the B area, free once
+    // every wave is past its MFMAs) so that each lane finishes whole outputs:
+    // row lane % 32 of the wave's 32, vectors lane / 32, + 2, ...  The
+    // three digit columns are combined once per output and each vector's 32
+    // rows leave as one 128-byte store.  Idle waves (rows past M) stay to the
+    // end for the block barriers.
+    __syncthreads();  // (10)
+    int *accs = reinterpret_cast<int *>(lds_b) + wave * (NMAT * 16 * 64);
+    if (wave_ok) {
 #pragma unroll
-    for (int i = 0; i < NMAT; ++i)
+      for (int i = 0; i < NMAT; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) accs[(i * 16 + r) * 64 + lane] = acc[i][r];
-  }
-  // accumulator element (row rl, column c) sits in register
-  // r = 4 (rl / 8) + rl % 4 of lane c + 32 ((rl / 4) % 2)
-  const int rl = lane & 31;
-  const int rr = 4 * (rl >> 3) + (rl & 3), lb = 32 * ((rl >> 2) & 1);
-  const int row = m0 + rl;
-  const bool row_live = wave_ok && row < a.M;
-  const int rowc = min(row, a.M - 1);
-  const float sc0 = a.scale[0][expert * a.s_stride + rowc];
-  const float sc1 = a.scale[NMAT - 1][expert * a.s_stride + rowc];
-  for (int t = lane >> 5; t < ti.ntok; t += 2) {
-    const int e = vexp[t];
-    const long long qsum = (long long)vsum[t];
-    float dot[NMAT];
+        for (int r = 0; r < 16; ++r) accs[(i * 16 + r) * 64 + lane] = acc[i][r];
+    }
+    // accumulator element (row n, column c) sits in register
+    // r = 4 (n / 8) + n % 4 of lane c + 32 ((n / 4) % 2)
+    const int rr = 4 * (n >> 3) + (n & 3), lb = 32 * ((n >> 2) & 1);
+    for (int t = h; t < ntok; t += 2) {
+      const int e = vexp[t];
+      const long long qsum = (long long)vsum[t];
+      float dot[NMAT];
 #pragma unroll
-    for (int i = 0; i < NMAT; ++i) {
-      const int *ar = accs + (i * 16 + rr) * 64 + lb + 3 * t;
-      const long long tot = (long long)ar[0] + ((long long)ar[1] << 8) + ((long long)ar[2] << 16);
-      dot[i] = e == kBadExp ? __builtin_nanf("") : (float)ldexp((double)(tot - qsum), -e);
+      for (int i = 0; i < NMAT; ++i) {
+        const int *ar = accs + (i * 16 + rr) * 64 + lb + 3 * t;
+        const long long tot = (long long)ar[0] + ((long long)ar[1] << 8) + ((long long)ar[2] << 16);
+        dot[i] = e == kBadExp ? __builtin_nanf("") : (float)ldexp((double)(tot - qsum), -e);
+      }
+      float y;
+      if constexpr (NMAT == 1) {
+        y = dot[0] * sc0;
+      } else {
+        const float g = dot[0] * sc0;
+        const float u = dot[1] * sc1;
+        y = (g * (1.0f / (1.0f + expf(-g)))) * u;
+      }
+      if (row_ok) {
+        a.out[(int64_t)vslot[t] * a.ld_out + row] = y;
+        if (a.out_max) atomicMax(&bmax[t], __float_as_uint(y) & 0x7fffffffu);  // LDS
+      }
     }
-    float y;
-    if constexpr (NMAT == 1) {
-      y = dot[0] * sc0;
-    } else {
-      const float g = dot[0] * sc0;
-      const float u = dot[1] * sc1;
-      y = (g * (1.0f / (1.0f + expf(-g)))) * u;
-    }
-    if (row_live) {
-      a.out[(int64_t)vslot[t] * a.ld_out + row] = y;
-      if (a.out_max) atomicMax(&bmax[t], __float_as_uint(y) & 0x7fffffffu);  // LDS
-    }
-  }
-  if (a.out_max) {  // this block's partial maximum per vector, no global atomics
-    __syncthreads();
-    if (tid < ti.ntok) a.out_max[(int64_t)vslot[tid] * gridDim.x + blockIdx.x] = bmax[tid];
-  }
+    if (a.out_max) __syncthreads();  // (11)
   }  // tiles of the block
 }
 
@@ -1102,6 +1139,7 @@ qmla_status qmla_packed_forward(const uint8_t *packed, const float *scales, int3
   QMLA_REQUIRE(scales != nullptr && x != nullptr && out != nullptr, QMLA_ERR_INVALID_ARG,
                "null pointer argument");
   PackedArgs a{};
+  a.early = 1;
   a.w[0] = a.w[1] = packed;
   a.scale[0] = a.scale[1] = scales;
   a.M = out_features;
@@ -1221,6 +1259,9 @@ qmla_status qmla_moe_forward(const qmla_moe_config *cfg, const float *xs, int32_
   gu.src_div = c.top_k;
   gu.ebin = block_bins ? nullptr : ebin;
   gu.slots = block_bins ? nullptr : slots;
+  // From one pair per two experts on, weights are requested at once; with
+  // fewer, the blocks without a token would take the others' bandwidth.
+  gu.early = 2 * (int64_t)P >= c.num_experts;
   gu.sel = block_bins && !rank_in_gemv ? sel : nullptr;
   gu.npairs = P;
   if (rank_in_gemv) {

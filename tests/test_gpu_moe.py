@@ -239,6 +239,26 @@ def test_moe_forward_skewed_routing(qmla_gpu, H, I):
 
 
 @pytest.mark.parametrize("E,k,H,I,T", [
+    (32, 4, 2048, 1408, 1), (32, 4, 2048, 1408, 5), (16, 1, 256, 512, 7), (16, 1, 256, 512, 8), (64, 8, 128, 1536, 3),
+    (3, 2, 4224, 4352, 2), (8, 2, 640, 1000, 11), (2, 1, 256, 256, 15)])
+def test_moe_gemv_edges(qmla_gpu, E, k, H, I, T):
+    """Fewer than eight pairs per expert: the GEMV path with its weights
+    requested before and after the bins are known (one pair per two experts),
+    bins of several tiles, row blocks past the last row, several slabs of K and
+    a per-row down product.  The sums are exact integers here; the oracle's four
+    f32 running sums of K / 4 <= 1088 products round by about 1088^0.5 2^-24 =
+    2e-6 in each of the two chained products, so 8e-6 bounds their maximum."""
+    q = qmla_gpu
+    W = O.random_moe_weights(E, k, H, I, 7500 + H + T)
+    xs = O.normal((T, H), 7600 + T)
+    out, idx, wts = moe_layer(q, W).forward(xs, return_routing=True)
+    ref, ridx, rw = O.moe_forward(W, xs, return_routing=True)
+    np.testing.assert_array_equal(idx, ridx)
+    np.testing.assert_allclose(wts, rw, rtol=1e-4, atol=1e-7)
+    assert rel_err(out, ref) < 8e-6
+
+
+@pytest.mark.parametrize("E,k,H,I,T", [
     (1, 1, 128, 128, 32), (2, 2, 128, 128, 33), (8, 2, 384, 640, 97), (5, 3, 1408, 2176, 50), (4, 4, 4224, 256, 9),
     (3, 1, 256, 384, 259)])
 def test_moe_grouped_edges(qmla_gpu, E, k, H, I, T):
