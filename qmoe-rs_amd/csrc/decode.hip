@@ -385,33 +385,50 @@ qmla_status validate_decode(const qmla_decode_dims *d, const qmla_kv_cache *c) {
 
 // Number of pieces: enough to fill the device, but no piece shorter than a
 // minimum so that per-piece overhead (q load, partial write) stays small.
-// 128 tokens (four 32-token tiles): at batch 1, 256 and 1024 cached tokens
-// step 2-3 us faster than with 256-token pieces; 64-token pieces make the
-// 4096-token step 6 us slower (the merge of 64 partials).
+// The MFMA plans count the virtual tokens they add per sequence: without them
+// 16 sequences of 100 tokens made 13 pieces of 444 virtual tokens, several
+// sequences to a piece.  f32: its 32-token tiles take 1.2 us each, so few
+// tokens go out one tile to a piece (278 tokens 27.8 us at 128 a piece, 14.1
+// at 32; 2222 tokens 28.3 and 17.3), for at most 32 rows and 64 sequences,
+// where the partials of 256 pieces stay below 22 MB.  bf16: two tiles (16
+// heads, 128 / 64 / 32 tokens a piece: 1 x 200 14.1 / 12.5 / 12.5 us, 1 x 4097
+// 15.3 / 14.8 / 17.8, 16 x 100 14.5 / 12.5 / 12.6; 128 heads, 1 x 500 21.8 /
+// 19.1 / 18.8, 4 x 1000 24.0 / 23.1 / 26.0).  The VALU path keeps 128.
+// This count sizes the workspace, so it never falls when lengths grow.
 int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t requested) {
   int64_t total = 0;
   for (int32_t i = 0; i < d->batch; ++i) total += c->h_lens[i];
   if (requested > 0) return std::min<int32_t>(requested, kMaxPlanBlocks);
   int cus = device_cu_count();
   if (cus <= 0) cus = 256;
-  int per_cu = (c->dtype == QMLA_BF16 && decode_mfma_supported(d->rows, d->kv_lora_rank, d->rope_dim))
-                   ? decode_mfma_blocks_per_cu(d->rows, d->kv_lora_rank, d->rope_dim)
-                   : decode_f32_blocks_per_cu(d->kv_lora_rank, d->rope_dim);
+  const bool bf16 = c->dtype == QMLA_BF16 && decode_mfma_supported(d->rows, d->kv_lora_rank, d->rope_dim);
+  int per_cu = bf16 ? decode_mfma_blocks_per_cu(d->rows, d->kv_lora_rank, d->rope_dim)
+                    : decode_f32_blocks_per_cu(d->kv_lora_rank, d->rope_dim);
   int64_t target = (int64_t)cus * per_cu;
   int64_t min_tokens = 128;
-  // The f32 MFMA decode reads its 32-token tiles at 1.2 us each, so few
-  // tokens go out one tile to a piece (counting the plan's virtual tokens):
-  // 278 tokens 27.8 us at 128 a piece, 14.1 at 32; 2222 tokens 28.3 and 17.3.
-  // At most 32 rows and 64 sequences, where the partials of 256 pieces stay
-  // below 22 MB.
-  if (c->dtype == QMLA_F32 && decode_f32_mfma_supported(d->kv_lora_rank, d->rope_dim) && d->rows <= 32 &&
-      d->batch <= 64) {
+  if (bf16) {
+    min_tokens = 64;
+    total += (int64_t)d->batch * decode_mfma_seg_tokens(d->rows, d->kv_lora_rank, d->rope_dim);
+  } else if (c->dtype == QMLA_F32 && decode_f32_mfma_supported(d->kv_lora_rank, d->rope_dim) &&
+             d->rows <= 32 && d->batch <= 64) {
     min_tokens = 32;
     total += (int64_t)d->batch * kDecodeF32SegTokens;
   }
   int64_t by_work = (total + min_tokens - 1) / min_tokens;
   int64_t blocks = std::max<int64_t>(1, std::min(target, by_work));
   return (int32_t)std::min<int64_t>(blocks, kMaxPlanBlocks);
+}
+
+// Pieces the bf16 plan launches of the `blocks` it may: pieces of two to four
+// tiles become whole tiles, since cut at 67 tokens some hold three tiles and
+// the rest two, with more partials to merge than pieces of three (16 heads, 4 x
+// 4000: 18.8 -> 16.7 us).
+int32_t whole_tile_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t blocks) {
+  int64_t total = (int64_t)d->batch * decode_mfma_seg_tokens(d->rows, d->kv_lora_rank, d->rope_dim);
+  for (int32_t i = 0; i < d->batch; ++i) total += c->h_lens[i];
+  const int64_t tiles = (total + 32LL * blocks - 1) / (32LL * blocks);
+  if (tiles < 2 || tiles > 4) return blocks;
+  return (int32_t)std::max<int64_t>(1, std::min<int64_t>(blocks, (total + 32 * tiles - 1) / (32 * tiles)));
 }
 
 qmla_status decode_impl(const qmla_decode_dims *d, const qmla_kv_cache *c, qmla_dtype q_dtype,
@@ -468,7 +485,7 @@ qmla_status qmla::decode_launch(const qmla_decode_dims *d, const qmla_kv_cache *
   a.seq_info = reinterpret_cast<int2 *>(ws);
   a.part_o = reinterpret_cast<float *>(static_cast<char *>(ws) + lay.part_o_off);
   a.part_lse = reinterpret_cast<float *>(static_cast<char *>(ws) + lay.part_lse_off);
-  a.blocks = blocks;
+  a.blocks = mfma && splits <= 0 ? whole_tile_blocks(d, c, blocks) : blocks;
   a.pending = pending;
   a.advance = advance;
   if (mfma) return launch_decode_mfma(a, s);  // decode + merge

@@ -856,6 +856,99 @@ __global__ __launch_bounds__(256) void k_decode_merge_frag(
   }
 }
 
+// The same merge with a column block's slots dealt to kMergeWaves waves, for
+// sequences of many slots: each wave merges its own, eight requested at a time,
+// and the waves' sums meet in LDS.  Slots enter in order within a wave, waves in
+// order after that.
+constexpr int kMergeWaves = 8;
+
+template <int R>
+__global__ __launch_bounds__(kMergeWaves * 64) void k_decode_merge_split(
+    int32_t rows, int32_t row_blocks, const int2 *__restrict__ seq_info,
+    const uint16_t *__restrict__ part_o, const float *__restrict__ part_lse, float *__restrict__ out,
+    float *__restrict__ out_lse, int32_t *__restrict__ adv_lens, int32_t adv, int32_t adv_n) {
+  constexpr int CB = R / 32, U = 8;
+  if (adv_lens && blockIdx.x == 0 && blockIdx.y == 0)
+    for (int i = threadIdx.x; i < adv_n; i += blockDim.x) adv_lens[i] += adv;
+  __shared__ float tile[kMergeWaves][32][33];
+  __shared__ float wave_mx[kMergeWaves][32], wave_sum[kMergeWaves][32];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int cb = blockIdx.y;
+  const int b = blockIdx.x / row_blocks, rb = blockIdx.x % row_blocks;
+  const int n = lane & 31, half = lane >> 5;
+  const int2 si = seq_info[b];
+  const int32_t sb = si.x, ns = si.y;
+  const int rows_pad = row_blocks * 32;
+  float acc[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+  float mx = -INFINITY, wsum = 0.f;
+  for (int k0 = wave; k0 < ns; k0 += kMergeWaves * U) {
+    float ls[U];
+    u32x2_t pv[U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // slots past the last re-read it, without weight
+      const int k = min(k0 + u * kMergeWaves, ns - 1);
+      ls[u] = part_lse[(int64_t)(sb + k) * rows_pad + rb * 32 + n];
+      const uint16_t *blk = part_o + (((int64_t)(sb + k) * row_blocks + rb) * CB + cb) * 1024 + lane * 4;
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) pv[u][jq] = *reinterpret_cast<const u32x2_t *>(blk + jq * 256);
+    }
+    float nm = mx;
+#pragma unroll
+    for (int u = 0; u < U; ++u) nm = fmaxf(nm, ls[u]);
+    const float ref = nm == -INFINITY ? 0.f : nm;  // no score yet: every weight is 0
+    const float alpha = expf(mx - ref);
+    mx = nm;
+    wsum *= alpha;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] *= alpha;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 + u * kMergeWaves >= ns) break;
+      const float w = expf(ls[u] - ref);
+      wsum += w;
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        acc[jq * 4 + 0] += w * __builtin_bit_cast(float, pv[u][jq][0] << 16);
+        acc[jq * 4 + 1] += w * __builtin_bit_cast(float, pv[u][jq][0] & 0xffff0000u);
+        acc[jq * 4 + 2] += w * __builtin_bit_cast(float, pv[u][jq][1] << 16);
+        acc[jq * 4 + 3] += w * __builtin_bit_cast(float, pv[u][jq][1] & 0xffff0000u);
+      }
+    }
+  }
+  if (half == 0) {
+    wave_mx[wave][n] = mx;
+    wave_sum[wave][n] = wsum;
+  }
+#pragma unroll
+  for (int jq = 0; jq < 4; ++jq)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tile[wave][n][8 * jq + 4 * half + e] = acc[jq * 4 + e];
+  __syncthreads();
+  // thread t: row t / 16, columns 2 (t % 16) and + 1
+  const int r = threadIdx.x >> 4, c = 2 * (threadIdx.x & 15);
+  const int row = rb * 32 + r;
+  if (row >= rows) return;
+  float m = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kMergeWaves; ++w) m = fmaxf(m, wave_mx[w][r]);
+  const float ref = m == -INFINITY ? 0.f : m;
+  float sum = 0.f, v0 = 0.f, v1 = 0.f;
+#pragma unroll
+  for (int w = 0; w < kMergeWaves; ++w) {
+    const float x = expf(wave_mx[w][r] - ref);
+    sum += x * wave_sum[w][r];
+    v0 += x * tile[w][r][c];
+    v1 += x * tile[w][r][c + 1];
+  }
+  const float inv = ns > 0 ? 1.f / sum : 0.f;
+  float *o = out + ((int64_t)b * rows + row) * R + cb * 32 + c;
+  o[0] = v0 * inv;
+  o[1] = v1 * inv;
+  if (cb == 0 && c == 0 && out_lse) out_lse[(int64_t)b * rows + row] = ns > 0 ? m + logf(sum) : -INFINITY;
+}
+
 // ---- narrow decode: one 32-row block (rows <= 32), all four SIMDs ------
 // With few query rows the MFMA work per token is small, so a block puts
 // four waves on one 32-row block instead of one wave: wave w computes S^T
@@ -1204,6 +1297,19 @@ __global__ __launch_bounds__(256) void k_decode_narrow(
 template <int R>
 qmla_status launch_merge(const DecodeArgs &a, hipStream_t stream) {
   const int row_blocks = (a.rows + 31) / 32;
+  // Slots per sequence (about blocks / batch) decide.  More than 16, past the
+  // plain merge's one round trip: 16 heads, 1 x 4097 27.6 -> 15.9 us (the whole
+  // call), 1 x 32768 79.0 -> 30.4, 4 x 1000 16.7 -> 13.0.  From 9 slots where the
+  // grid is at most two blocks per CU: 128 heads, 8 x 1000 27.0 -> 25.1, but 16 x
+  // 4000 44.0 -> 45.1.  At fewer the LDS round is not won back: 1 x 40 11.4 ->
+  // 12.8, 16 x 100 12.4 -> 13.6.
+  if (a.blocks > (a.batch * row_blocks <= 32 ? 8 : 16) * a.batch) {
+    k_decode_merge_split<R><<<dim3((unsigned)(a.batch * row_blocks), R / 32), dim3(kMergeWaves * 64), 0, stream>>>(
+        a.rows, row_blocks, a.seq_info, (const uint16_t *)a.part_o, a.part_lse, a.out, a.out_lse,
+        a.advance ? a.cache->d_lens : nullptr, a.pending, a.batch);
+    QMLA_LAUNCH_CHECK("k_decode_merge_split");
+    return QMLA_OK;
+  }
   dim3 mgrid((unsigned)(a.batch * row_blocks), (R / 32 + 3) / 4);
   k_decode_merge_frag<R><<<mgrid, dim3(256), 0, stream>>>(
       a.rows, row_blocks, a.seq_info, (const uint16_t *)a.part_o, a.part_lse, a.out, a.out_lse,

@@ -339,3 +339,27 @@ def test_decode_f32_mfma_large_batch(qmla_gpu):
         assert rel_err(out, ref) < 2e-5
         assert np.all(out[~live] == 0) and np.all(np.isneginf(lse[~live]))
         np.testing.assert_allclose(lse[live], rlse[live], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("rows_m,r,dr", [(16, 512, 64), (33, 512, 64), (128, 512, 64), (48, 64, 16)])
+@pytest.mark.parametrize("lens", [[3001], [31, 0, 700, 33, 64, 65, 1900], [0] + [97] * 20])
+def test_decode_bf16_piece_counts_and_merges(qmla_gpu, rows_m, r, dr, lens):
+    """Pieces of two tiles and more, one to dozens of partial slots per
+    sequence on either merge, empty sequences; and a workspace sized while the
+    sequences were longer serves the shorter ones."""
+    q = qmla_gpu
+    cache, rows, offs = make_cache(q, lens, r, dr, q.BF16, 1700 + rows_m)
+    b = len(lens)
+    ql, qr = O.normal((b, rows_m, r), 1701), O.normal((b, rows_m, dr), 1702)
+    need = q.decode_workspace_bytes(cache, b, rows_m)
+    for cut in (1.0, 0.6):
+        now = np.asarray([int(n * cut) for n in lens], np.int32)
+        cache.set_lengths(now)
+        assert q.decode_workspace_bytes(cache, b, rows_m) <= need
+        ref, rlse = O.decode_absorbed(ql, qr, rows, offs, now, 0.06)
+        live = now > 0
+        for splits in (0, 1, 9 * b, 200):
+            out, lse = run(q, cache, ql, qr, 0.06, splits=splits)
+            assert rel_err(out, ref) < TOL_BF16
+            assert np.all(out[~live] == 0) and np.all(np.isneginf(lse[~live]))
+            np.testing.assert_allclose(lse[live], rlse[live], atol=2e-2)
