@@ -179,9 +179,41 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
       }
     }
   };
+  // What the epilogue of pair e (outputs j, j + 1 of lane l = e % 64) needs
+  // from memory: its biases and, for a rope pair, position and frequency.
+  struct Pre {
+    float b0, b1, pos, freq;
+  };
+  const float *bias = a.bias && grp == 0 ? a.bias + z * a.sb : nullptr;
+  const int qw = a.dn + a.dr, hq = a.heads * qw;
+  auto prefetch = [&](int e) __attribute__((always_inline)) {
+    Pre p{0.f, 0.f, 0.f, 0.f};
+    const int j = 2 * (e >> 6), l = e & 63, m = l & 31;
+    const int n = n0 + 8 * (j >> 2) + 4 * (l >> 5) + (j & 3);  // even
+    if (m >= a.M || n >= a.N) return p;
+    if (bias) {
+      p.b0 = bias[n];
+      if (n + 1 < a.N) p.b1 = bias[n + 1];
+    }
+    if (a.mode == kSkinnyQkv && n < hq && n % qw >= a.dn) {
+      const int b = (a.m0 + m) / a.seq;
+      p.pos = (float)(a.lens[b] + (a.m0 + m - b * a.seq));
+      p.freq = a.inv_freq[(n % qw - a.dn) >> 1];
+    }
+    return p;
+  };
+  // Eight waves: one pair per thread, requested ahead of the weights and
+  // turned into the rotation under their latency (one user's step 45.4 -> 44.1
+  // us; after the reduction these were two more round trips).
+  constexpr bool kAhead = NW == 8;
+  Pre ahead{};
+  float cs_a = 0.f, sn_a = 0.f;
+  if constexpr (kAhead) ahead = prefetch(threadIdx.x);
   // two chunks in flight: the loads of chunk i + 1 go out before the MFMAs
   // of chunk i
   load(0, 0);
+  if constexpr (kAhead)
+    if (a.mode == kSkinnyQkv) rope_cs(ahead.pos * ahead.freq, a.mscale, cs_a, sn_a);
   int s0 = 0;
   for (; s0 + 2 * kChunk < steps; s0 += 2 * kChunk) {
     load(1, s0 + kChunk);
@@ -200,10 +232,10 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
 #pragma unroll
   for (int j = 0; j < 16; ++j) red[wave][j][lane] = acc[j];
   __syncthreads();
-  const float *bias = a.bias && grp == 0 ? a.bias + z * a.sb : nullptr;
   // epilogue over pairs (j, j + 1), j even: adjacent outputs of one token
   for (int e = threadIdx.x; e < 8 * 64; e += NW * 64) {
     const int j = 2 * (e >> 6), l = e & 63;
+    const Pre pre = kAhead ? ahead : prefetch(e);
     float v0 = 0.f, v1 = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
@@ -214,8 +246,8 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
     const int n = n0 + 8 * (j >> 2) + 4 * (l >> 5) + (j & 3);  // even
     if (m >= a.M || n >= a.N) continue;
     if (bias) {
-      v0 += bias[n];
-      if (n + 1 < a.N) v1 += bias[n + 1];
+      v0 += pre.b0;
+      v1 += pre.b1;
     }
     if (a.mode == kSkinnyFinal) {
       float *y = a.y + z * a.sy + grp * a.sgrp + (int64_t)m * a.ldy + n;
@@ -238,7 +270,6 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
       continue;
     }
     // kSkinnyQkv: n in [0, H (dn + dr)) is q_proj's output, the rest kv_a
-    const int qw = a.dn + a.dr, hq = a.heads * qw;
     const int mg = a.m0 + m;  // token index in the whole call
     if (n >= hq) {
       float *y = (grp ? a.kva1 : a.kva) + (int64_t)mg * a.kva_ld + (n - hq);
@@ -255,11 +286,8 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
       // interleaved pair (2p, 2p + 1) of q_rope (src/model.rs:70-84); the
       // rotation is linear, so each K-half is rotated on its own
       const int p = (d - a.dn) >> 1;
-      const int b = mg / a.seq, i = mg - b * a.seq;
-      const float pos = (float)(a.lens[b] + i);
-      const float ang = pos * a.inv_freq[p];
-      float cs, sn;
-      rope_cs(ang, a.mscale, cs, sn);
+      float cs = cs_a, sn = sn_a;
+      if constexpr (!kAhead) rope_cs(pre.pos * pre.freq, a.mscale, cs, sn);
       float *y = (grp ? a.q_rope1 : a.q_rope) + ((int64_t)mg * a.heads + hd) * a.dr + 2 * p;
       y[0] = v0 * cs - v1 * sn;
       y[1] = v1 * cs + v0 * sn;

@@ -215,6 +215,35 @@ def test_prefill_rows_gemm(qmla_gpu, dt, dims, b, s):
     assert rel_err(layer.forward_with_cache(x1, cache), ref1) < (TOL if dt == "f32" else 2e-2)
 
 
+@pytest.mark.parametrize("dims,dt", [
+    # hidden, heads, qk_nope, qk_rope, v_dim, kv_lora_rank
+    ((128, 2, 32, 128, 32, 64), "f32"),  # rope as wide as one wave takes
+    ((128, 2, 32, 16, 32, 520), "f32"),  # latents past one wave: the block's row kernel
+    ((128, 4, 32, 20, 32, 68), "f32"),   # widths that are no multiple of 8: the same
+    ((128, 2, 32, 16, 32, 64), "bf16"),
+    ((512, 4, 128, 64, 128, 512), "f32"),
+    ((512, 4, 128, 64, 128, 512), "bf16"),
+])
+def test_decode_new_rows_at_their_positions(qmla_gpu, dims, dt):
+    """The new tokens' cache rows of decode steps (LayerNorm, RoPE, two tokens a
+    step) on the one-wave and the block row kernel, through the attention over
+    them against the oracle's (f32: 1e-4)."""
+    q = qmla_gpu
+    hidden, H, dn, dr, dv, r = dims
+    w = O.MlaWeights.random(hidden, H, dn, dr, dv, r, seed=2400 + r + dr)
+    layer = q.MlaLayer(w)
+    b = 3
+    xs = O.normal((b, 9, hidden), 2401)
+    cache = q.KVCache([16] * b, r, dr, q.F32 if dt == "f32" else q.BF16)
+    layer.forward_prefill(xs, cache)
+    _, (k, v, kr) = O.mla_forward_prefill(w, xs)
+    for step in range(2):
+        x = O.normal((b, 2, hidden), 2410 + step)
+        out = layer.forward_with_cache(x, cache)
+        ref, (k, v, kr) = O.mla_forward_with_cache(w, x, k, v, kr, return_cache=True)
+        assert rel_err(out, ref) < (TOL if dt == "f32" else 2e-2)
+
+
 def _ragged_cache(q, lens, r, dr, dtype, seed, spare=2):
     """A cache whose sequences hold `lens` random latent rows (N(0,1); bf16
     rounded for a bf16 cache) with `spare` free rows each; returns the cache
