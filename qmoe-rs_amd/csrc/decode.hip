@@ -395,7 +395,10 @@ qmla_status validate_decode(const qmla_decode_dims *d, const qmla_kv_cache *c) {
 // 15.3 / 14.8 / 17.8, 16 x 100 14.5 / 12.5 / 12.6; 128 heads, 1 x 500 21.8 /
 // 19.1 / 18.8, 4 x 1000 24.0 / 23.1 / 26.0).  The VALU path keeps 128.
 // This count sizes the workspace, so it never falls when lengths grow.
-int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t requested) {
+// `coarse`: pieces of 128 tokens on every path, for the fixed scratch where it
+// holds no more.
+int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t requested,
+                      bool coarse = false) {
   int64_t total = 0;
   for (int32_t i = 0; i < d->batch; ++i) total += c->h_lens[i];
   if (requested > 0) return std::min<int32_t>(requested, kMaxPlanBlocks);
@@ -406,10 +409,10 @@ int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t
                     : decode_f32_blocks_per_cu(d->kv_lora_rank, d->rope_dim);
   int64_t target = (int64_t)cus * per_cu;
   int64_t min_tokens = 128;
-  if (bf16) {
+  if (bf16 && !coarse) {
     min_tokens = 64;
     total += (int64_t)d->batch * decode_mfma_seg_tokens(d->rows, d->kv_lora_rank, d->rope_dim);
-  } else if (c->dtype == QMLA_F32 && decode_f32_mfma_supported(d->kv_lora_rank, d->rope_dim) &&
+  } else if (!coarse && c->dtype == QMLA_F32 && decode_f32_mfma_supported(d->kv_lora_rank, d->rope_dim) &&
              d->rows <= 32 && d->batch <= 64) {
     min_tokens = 32;
     total += (int64_t)d->batch * kDecodeF32SegTokens;
@@ -543,18 +546,24 @@ qmla_status qmla_decode_absorbed_noalloc(const qmla_decode_dims *dims, const qml
                                          const void *q_rope, double scale, float *out_latent,
                                          float *out_lse, qmla_stream stream) {
   QMLA_TRY(validate_decode(dims, cache));
-  const int32_t blocks = choose_blocks(dims, cache, 0);
-  const size_t need = decode_workspace_layout(dims->batch, dims->rows, dims->kv_lora_rank, blocks,
-                                              cache->dtype == QMLA_BF16)
-                          .total;
+  // the pieces of the workspace entry point where the scratch holds their
+  // partials, else pieces of 128 tokens
+  auto need_of = [&](int32_t blocks) {
+    return decode_workspace_layout(dims->batch, dims->rows, dims->kv_lora_rank, blocks,
+                                   cache->dtype == QMLA_BF16)
+        .total;
+  };
+  const int32_t coarse = choose_blocks(dims, cache, 0, /*coarse=*/true);
+  const size_t need = need_of(coarse);
   QMLA_REQUIRE(need <= kNoAllocScratchBytes, QMLA_ERR_UNSUPPORTED,
                "decode needs %zu bytes of scratch; the allocation-free entry point has %zu "
                "(use qmla_decode_absorbed with a workspace)",
                need, kNoAllocScratchBytes);
+  const int32_t splits = need_of(choose_blocks(dims, cache, 0)) <= kNoAllocScratchBytes ? 0 : coarse;
   void *ws = nullptr;
   QMLA_TRY(noalloc_scratch(&ws));
-  return decode_impl(dims, cache, q_dtype, q_latent, q_rope, scale, out_latent, out_lse, 0, ws,
-                     kNoAllocScratchBytes, stream);
+  return decode_impl(dims, cache, q_dtype, q_latent, q_rope, scale, out_latent, out_lse,
+                     splits, ws, kNoAllocScratchBytes, stream);
 }
 
 qmla_status qmla_decode_workspace_bytes_splits(const qmla_decode_dims *dims,
