@@ -26,9 +26,9 @@
  *    one GPU race and must be serialised by the caller).  Every other call
  *    on different streams may run from different threads.  A cache object
  *    must not be mutated concurrently.
- *    A layer object may be used from several threads at once: its GEMM path
- *    (prefill, and decode shapes the skinny kernel does not take) takes one
- *    of 4 rocBLAS handles created with the layer, so up to 4 such calls run
+ *    A layer object may be used from several threads at once: its rocBLAS
+ *    path (shapes the hand-written projections do not take) takes one of 4
+ *    handles created with the layer, so up to 4 such calls run
  *    without waiting for each other.
  */
 #ifndef QMLA_H
@@ -342,8 +342,9 @@ QMLA_API qmla_status qmla_layer_destroy(qmla_layer *layer);
  *     bf16 (their hi halves), the activations rounded to nearest even; one
  *     MFMA per step and half the weight bytes.  Results then hold the bf16
  *     tolerance (2e-2), whatever the cache dtype.
- * The rocBLAS paths (prefill below 128 tokens, decode shapes the skinny
- * kernel does not take) and qmla_cache_materialise stay f32-exact.  Applies
+ * A prefill below 128 tokens (f32 products), the rocBLAS paths (shapes the
+ * hand-written projections do not take) and qmla_cache_materialise stay
+ * f32-exact.  Applies
  * to calls issued after it returns: set it before the layer is shared with
  * other threads.  QMLA_ERR_INVALID_ARG for a NULL layer or another dtype. */
 QMLA_API qmla_status qmla_layer_set_projection_dtype(qmla_layer *layer, qmla_dtype dtype);
