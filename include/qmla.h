@@ -268,6 +268,8 @@ typedef struct {
   int32_t rope_dim;     /* must equal the cache's                       */
 } qmla_decode_dims;
 
+/* Scratch of qmla_decode_absorbed at the cache's current lengths.  It also
+ * serves every call of fewer sequences, fewer rows or shorter sequences.   */
 QMLA_API qmla_status qmla_decode_workspace_bytes(const qmla_decode_dims *dims, const qmla_kv_cache *cache,
                                         size_t *bytes);
 QMLA_API qmla_status qmla_decode_absorbed(const qmla_decode_dims *dims, const qmla_kv_cache *cache,

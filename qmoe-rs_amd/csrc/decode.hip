@@ -394,7 +394,8 @@ qmla_status validate_decode(const qmla_decode_dims *d, const qmla_kv_cache *c) {
 // heads, 128 / 64 / 32 tokens a piece: 1 x 200 14.1 / 12.5 / 12.5 us, 1 x 4097
 // 15.3 / 14.8 / 17.8, 16 x 100 14.5 / 12.5 / 12.6; 128 heads, 1 x 500 21.8 /
 // 19.1 / 18.8, 4 x 1000 24.0 / 23.1 / 26.0).  The VALU path keeps 128.
-// This count sizes the workspace, so it never falls when lengths grow.
+// The count never falls when lengths grow; workspace_bytes_auto below makes the
+// workspace's size grow with rows and batch too.
 // `coarse`: pieces of 128 tokens on every path, for the fixed scratch where it
 // holds no more.
 int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t requested,
@@ -432,6 +433,24 @@ int32_t whole_tile_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int
   const int64_t tiles = (total + 32LL * blocks - 1) / (32LL * blocks);
   if (tiles < 2 || tiles > 4) return blocks;
   return (int32_t)std::max<int64_t>(1, std::min<int64_t>(blocks, (total + 32 * tiles - 1) / (32 * tiles)));
+}
+
+// Workspace of an automatic split: what the call itself needs, or a call of
+// fewer rows or sequences over the same cache, whichever is more.  The piece
+// count depends on the row class (up to 32, up to 64, more) and in f32 on the
+// batch (up to 64, more), and steps down where a class ends: 65 sequences x 100
+// tokens of 16 rows make 51 pieces in f32, 64 of them 256.  Within a class the
+// size grows with every dimension, so the largest call of each class bounds it.
+size_t workspace_bytes_auto(const qmla_decode_dims *d, const qmla_kv_cache *c) {
+  size_t need = 0;
+  for (int32_t rows : {32, 64, d->rows})
+    for (int32_t batch : {64, d->batch}) {
+      const qmla_decode_dims e{std::min(batch, d->batch), std::min(rows, d->rows), d->kv_lora_rank, d->rope_dim};
+      need = std::max(need, decode_workspace_layout(e.batch, e.rows, e.kv_lora_rank, choose_blocks(&e, c, 0),
+                                                    c->dtype == QMLA_BF16)
+                                .total);
+    }
+  return need;
 }
 
 qmla_status decode_impl(const qmla_decode_dims *d, const qmla_kv_cache *c, qmla_dtype q_dtype,
@@ -572,6 +591,10 @@ qmla_status qmla_decode_workspace_bytes_splits(const qmla_decode_dims *dims,
   QMLA_REQUIRE(bytes, QMLA_ERR_INVALID_ARG, "bytes is NULL");
   QMLA_TRY(validate_decode(dims, cache));
   QMLA_REQUIRE(num_splits >= 0, QMLA_ERR_INVALID_ARG, "negative split count");
+  if (num_splits == 0) {
+    *bytes = workspace_bytes_auto(dims, cache);
+    return QMLA_OK;
+  }
   int32_t blocks = choose_blocks(dims, cache, num_splits);
   *bytes = decode_workspace_layout(dims->batch, dims->rows, dims->kv_lora_rank, blocks,
                                    cache->dtype == QMLA_BF16)

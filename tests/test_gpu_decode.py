@@ -363,3 +363,26 @@ def test_decode_bf16_piece_counts_and_merges(qmla_gpu, rows_m, r, dr, lens):
             assert rel_err(out, ref) < TOL_BF16
             assert np.all(out[~live] == 0) and np.all(np.isneginf(lse[~live]))
             np.testing.assert_allclose(lse[live], rlse[live], atol=2e-2)
+
+
+@pytest.mark.parametrize("dt,lens,rows_m,fewer", [
+    ("f32", [100] * 65, 16, (64, 16)), ("f32", [300] * 8, 48, (8, 16)), ("f32", [5] * 70, 33, (3, 1)),
+    ("bf16", [2000] * 16, 80, (16, 64)), ("bf16", [10] * 40, 48, (40, 16)), ("bf16", [700] * 3, 128, (2, 33))])
+def test_decode_workspace_serves_fewer_rows_and_sequences(qmla_gpu, dt, lens, rows_m, fewer):
+    """A workspace sized once for the largest step serves every smaller one:
+    the piece count steps up where a class of rows or batches ends."""
+    q = qmla_gpu
+    cache, rows, offs = make_cache(q, lens, 512, 64, q.F32 if dt == "f32" else q.BF16, 1900 + rows_m)
+    need = q.decode_workspace_bytes(cache, len(lens), rows_m)
+    for b in {1, fewer[0], len(lens)}:
+        for m in {1, 32, fewer[1], 64, 65, rows_m}:
+            if m <= rows_m:
+                assert q.decode_workspace_bytes(cache, b, m) <= need
+    b, m = fewer
+    ql, qr = O.normal((b, m, 512), 1901), O.normal((b, m, 64), 1902)
+    dql, dqr = q.DeviceBuffer.from_numpy(ql), q.DeviceBuffer.from_numpy(qr)
+    out, ws = q.DeviceBuffer(b * m * 512 * 4), q.DeviceBuffer(need)
+    q.decode_absorbed(cache, b, m, dql, dqr, 0.07, out, workspace=ws, workspace_bytes=need)
+    q.check(q.lib().qmla_stream_synchronize(None))
+    ref, _ = O.decode_absorbed(ql[:3], qr[:3], rows, offs[:3], np.asarray(lens[:3], np.int32), 0.07)
+    assert rel_err(out.to_numpy(np.float32, (b, m, 512))[:3], ref) < (TOL_F32 if dt == "f32" else TOL_BF16)
