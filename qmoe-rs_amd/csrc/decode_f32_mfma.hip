@@ -296,6 +296,8 @@ __global__ __launch_bounds__(512) void k_decode_merge_f32(int32_t rows, const in
 bool decode_f32_mfma_supported(int32_t r, int32_t dr) { return r == kR && dr == kDr; }
 
 qmla_status launch_decode_f32_mfma(const DecodeArgs &a, hipStream_t stream) {
+  // the merge's grid has a row per query row
+  QMLA_REQUIRE(a.rows <= 65535, QMLA_ERR_SHAPE, "rows %d > 65535", a.rows);
   const dim3 grid(a.blocks, (a.rows + kRowsPerBlock - 1) / kRowsPerBlock);
   const PageTable tab = a.cache->table();
   if (a.q_dtype == QMLA_BF16) {

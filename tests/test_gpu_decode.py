@@ -386,3 +386,20 @@ def test_decode_workspace_serves_fewer_rows_and_sequences(qmla_gpu, dt, lens, ro
     q.check(q.lib().qmla_stream_synchronize(None))
     ref, _ = O.decode_absorbed(ql[:3], qr[:3], rows, offs[:3], np.asarray(lens[:3], np.int32), 0.07)
     assert rel_err(out.to_numpy(np.float32, (b, m, 512))[:3], ref) < (TOL_F32 if dt == "f32" else TOL_BF16)
+
+
+@pytest.mark.parametrize("r,dr", [(512, 64), (64, 16)])
+def test_decode_f32_refuses_more_rows_than_the_merge_grid(qmla_gpu, r, dr):
+    """65536 query rows: QMLA_ERR_SHAPE on either f32 kernel, with the output
+    untouched."""
+    q = qmla_gpu
+    m = 65536
+    cache, _, _ = make_cache(q, [1], r, dr, q.F32, 1950)
+    ql, qr = q.DeviceBuffer(m * r * 4), q.DeviceBuffer(m * dr * 4)
+    out = q.DeviceBuffer.from_numpy(np.full((m, r), 7.0, np.float32))
+    need = q.decode_workspace_bytes(cache, 1, m)
+    ws = q.DeviceBuffer(need)
+    with pytest.raises(q.QmlaError) as e:
+        q.decode_absorbed(cache, 1, m, ql, qr, 0.1, out, workspace=ws, workspace_bytes=need)
+    assert e.value.status == 2
+    assert (out.to_numpy(np.float32, (m, r)) == 7.0).all()
