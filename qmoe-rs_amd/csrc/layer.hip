@@ -752,11 +752,15 @@ LayerWs layer_ws(const qmla_layer *L, int32_t batch, int32_t seq, size_t dec_byt
   // o: [n][H dv] f32, or o_proj's packed B operand of 32 token rows (the
   // same 4 bytes per element, 32 rows at least)
   w.o = take(sizeof(float) * std::max<size_t>(n, 32) * H * g.v_dim);
-  // split-K partials of the skinny projections (16 slices at most)
+  // split-K partials of the skinny projections and of rocBLAS below 64 rows
+  // (16 slices at most).  More rows use none, but keep the region, so that a
+  // workspace sized for them serves fewer.  Hand-written prefills have their
+  // own (sgpart).
   const size_t widest = std::max<size_t>({(size_t)H * (g.qk_nope + g.qk_rope),
                                           (size_t)(g.kv_lora_rank + g.qk_rope), (size_t)g.hidden});
-  w.part_elems = n <= (size_t)kSkinnyRows ? 16 * n * widest : 0;
-  w.part = take(sizeof(float) * (w.part_elems ? w.part_elems : 1));
+  const size_t few = std::min(n, (size_t)kSkinnyRows);
+  w.part_elems = n <= (size_t)kSkinnyRows && !sg_only ? 16 * n * widest : 0;
+  w.part = take(sg_only ? 1 : sizeof(float) * 16 * few * widest);
   // bf16 halves of a projection's activations (rocBLAS split GEMMs, many rows)
   const size_t kmax = std::max<size_t>({(size_t)g.hidden, H * g.v_dim, (size_t)g.kv_lora_rank});
   w.xsplit =
@@ -768,11 +772,10 @@ LayerWs layer_ws(const qmla_layer *L, int32_t batch, int32_t seq, size_t dec_byt
     w.olat = take(sizeof(float) * n * H * g.kv_lora_rank);
     w.dec = take(dec_bytes);
     // the second K-half of the skinny q_proj | kv_a product
-    if (n <= (size_t)kSkinnyRows) {
-      w.qn1 = take(sizeof(float) * n * H * g.qk_nope);
-      w.qr1 = take(sizeof(float) * n * H * g.qk_rope);
-      w.kva1 = take(sizeof(float) * n * (g.kv_lora_rank + g.qk_rope));
-    }
+    // (kept beyond kSkinnyRows rows, as part)
+    w.qn1 = take(sizeof(float) * few * H * g.qk_nope);
+    w.qr1 = take(sizeof(float) * few * H * g.qk_rope);
+    w.kva1 = take(sizeof(float) * few * (g.kv_lora_rank + g.qk_rope));
     dec_end = off;
   }
   if (use != WsFor::kDecode) {
@@ -801,6 +804,9 @@ LayerWs layer_ws(const qmla_layer *L, int32_t batch, int32_t seq, size_t dec_byt
     pre_end = off;
   }
   w.total = std::max(dec_end, pre_end);
+  // the K-slice partials of the rows GEMM can be more than the split GEMM's
+  if (sg && use != WsFor::kDecode)
+    w.total = std::max(w.total, layer_ws(L, 1, kSplitGemmMinRows - 1, 0, WsFor::kPrefill).total);
   return w;
 }
 

@@ -682,3 +682,22 @@ def test_layer_bf16_projections_at_small_latent_dims(qmla_gpu, b, s):
     assert err < 2e-2 and err1 < 2e-2
     with pytest.raises(q.QmlaError):
         layer.set_projection_dtype(7)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("hidden,H,dn,dr,dv,r", [(512, 16, 128, 64, 128, 512), (256, 4, 32, 16, 32, 64)])
+def test_layer_workspace_serves_fewer_tokens(qmla_gpu, dt, hidden, H, dn, dr, dv, r):
+    """A workspace sized for a prompt or step serves every shorter one, across
+    the sizes at which the projections change kernels (64, 128 rows)."""
+    q = qmla_gpu
+    layer = q.MlaLayer(O.MlaWeights.random(hidden, H, dn, dr, dv, r, seed=1950))
+    cache = q.KVCache([512] * 200, r, dr, q.F32 if dt == "f32" else q.BF16)
+    short = [1, 7, 32, 33, 63, 64, 65, 66, 100, 126, 127]
+    for long in short + [128, 129, 140, 200, 300]:
+        pre, step = layer.prefill_workspace_bytes(cache, 1, long), layer.workspace_bytes(cache, 1, long)
+        for n in short:
+            if n < long:
+                assert layer.prefill_workspace_bytes(cache, 1, n) <= pre, (n, long)
+                assert layer.workspace_bytes(cache, 1, n) <= step, (n, long)
+    steps = [layer.workspace_bytes(cache, b, 1) for b in (1, 31, 32, 33, 63, 64, 65, 66, 100, 127, 128, 200)]
+    assert steps == sorted(steps)
