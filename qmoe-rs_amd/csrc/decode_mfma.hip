@@ -1391,9 +1391,13 @@ bool decode_narrow_path(int32_t rows, int32_t r, int32_t dr) {
   return rows <= 32 && r == 512 && dr == 64;
 }
 
+// Rank 512 has one block per compute unit at any row count (its tile ring is
+// 110 KB of LDS or more).  Two pieces per unit, which 33 .. 64 rows once had,
+// ran as a second round: 48 rows, 512 / 256 pieces, 16 x 4000 48.7 / 33.2 us,
+// 64 x 500 42.6 / 29.2.
 int decode_mfma_blocks_per_cu(int32_t rows, int32_t r, int32_t dr) {
   if (decode_narrow_path(rows, r, dr)) return 1;
-  return rows <= 64 ? 2 : 1;
+  return rows <= 64 && r < 512 ? 2 : 1;
 }
 
 // Virtual tokens charged per sequence start in the split plan: the fixed

@@ -403,3 +403,19 @@ def test_decode_f32_refuses_more_rows_than_the_merge_grid(qmla_gpu, r, dr):
         q.decode_absorbed(cache, 1, m, ql, qr, 0.1, out, workspace=ws, workspace_bytes=need)
     assert e.value.status == 2
     assert (out.to_numpy(np.float32, (m, r)) == 7.0).all()
+
+
+@pytest.mark.parametrize("rows_m", [33, 48, 64])
+def test_decode_bf16_one_piece_per_compute_unit_at_rank_512(qmla_gpu, rows_m):
+    """A block of 33 .. 64 rows fills a compute unit's LDS: more pieces than
+    units run as a second round.  At every length the automatic split takes no
+    more, and the result is the oracle's."""
+    q = qmla_gpu
+    cus = q.device_info()[1]
+    lens = [32 * 1024, 40 * 1024, 100]
+    cache, rows, offs = make_cache(q, lens, 512, 64, q.BF16, 1960)
+    assert q.decode_workspace_bytes(cache, 3, rows_m) <= q.decode_workspace_bytes(cache, 3, rows_m, splits=cus)
+    ql, qr = O.normal((3, rows_m, 512), 1961), O.normal((3, rows_m, 64), 1962)
+    out, _ = run(q, cache, ql, qr, 0.06)
+    ref, _ = O.decode_absorbed(ql, qr, rows, offs, np.asarray(lens, np.int32), 0.06)
+    assert rel_err(out, ref) < TOL_BF16
