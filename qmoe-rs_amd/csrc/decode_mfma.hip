@@ -856,15 +856,17 @@ __global__ __launch_bounds__(256) void k_decode_merge_frag(
   }
 }
 
-// The same merge with a column block's slots dealt to kMergeWaves waves, for
-// sequences of many slots: each wave merges its own, eight requested at a time,
-// and the waves' sums meet in LDS.  Slots enter in order within a wave, waves in
-// order after that.
+// The same merge for batches that hold sequences of many slots.  Sequences of
+// more than `few` slots deal a column block's slots to kMergeWaves waves: each
+// merges its own, eight requested at a time, and the waves' sums meet in LDS.
+// Slots enter in order within a wave, waves in order after that.  The others
+// take a column block per wave, in the blocks of every kMergeWaves-th column
+// block; the rest of theirs have nothing to do.
 constexpr int kMergeWaves = 8;
 
 template <int R>
 __global__ __launch_bounds__(kMergeWaves * 64) void k_decode_merge_split(
-    int32_t rows, int32_t row_blocks, const int2 *__restrict__ seq_info,
+    int32_t rows, int32_t row_blocks, int32_t few, const int2 *__restrict__ seq_info,
     const uint16_t *__restrict__ part_o, const float *__restrict__ part_lse, float *__restrict__ out,
     float *__restrict__ out_lse, int32_t *__restrict__ adv_lens, int32_t adv, int32_t adv_n) {
   constexpr int CB = R / 32, U = 8;
@@ -873,22 +875,25 @@ __global__ __launch_bounds__(kMergeWaves * 64) void k_decode_merge_split(
   __shared__ float tile[kMergeWaves][32][33];
   __shared__ float wave_mx[kMergeWaves][32], wave_sum[kMergeWaves][32];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int cb = blockIdx.y;
   const int b = blockIdx.x / row_blocks, rb = blockIdx.x % row_blocks;
   const int n = lane & 31, half = lane >> 5;
   const int2 si = seq_info[b];
   const int32_t sb = si.x, ns = si.y;
+  const bool solo = ns <= few;
+  const int cb = blockIdx.y + (solo ? wave : 0);
+  if (solo && (blockIdx.y % kMergeWaves != 0 || cb >= CB)) return;
+  const int first = solo ? 0 : wave, step = solo ? 1 : kMergeWaves;
   const int rows_pad = row_blocks * 32;
   float acc[16];
 #pragma unroll
   for (int j = 0; j < 16; ++j) acc[j] = 0.f;
   float mx = -INFINITY, wsum = 0.f;
-  for (int k0 = wave; k0 < ns; k0 += kMergeWaves * U) {
+  for (int k0 = first; k0 < ns; k0 += step * U) {
     float ls[U];
     u32x2_t pv[U][4];
 #pragma unroll
     for (int u = 0; u < U; ++u) {  // slots past the last re-read it, without weight
-      const int k = min(k0 + u * kMergeWaves, ns - 1);
+      const int k = min(k0 + u * step, ns - 1);
       ls[u] = part_lse[(int64_t)(sb + k) * rows_pad + rb * 32 + n];
       const uint16_t *blk = part_o + (((int64_t)(sb + k) * row_blocks + rb) * CB + cb) * 1024 + lane * 4;
 #pragma unroll
@@ -905,7 +910,7 @@ __global__ __launch_bounds__(kMergeWaves * 64) void k_decode_merge_split(
     for (int j = 0; j < 16; ++j) acc[j] *= alpha;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (k0 + u * kMergeWaves >= ns) break;
+      if (k0 + u * step >= ns) break;
       const float w = expf(ls[u] - ref);
       wsum += w;
 #pragma unroll
@@ -916,6 +921,28 @@ __global__ __launch_bounds__(kMergeWaves * 64) void k_decode_merge_split(
         acc[jq * 4 + 3] += w * __builtin_bit_cast(float, pv[u][jq][1] & 0xffff0000u);
       }
     }
+  }
+  if (solo) {
+    const float inv = ns > 0 ? 1.f / wsum : 0.f;
+    if (cb == 0 && half == 0 && out_lse && rb * 32 + n < rows)
+      out_lse[(int64_t)b * rows + rb * 32 + n] = ns > 0 ? mx + logf(wsum) : -INFINITY;
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tile[wave][n][8 * jq + 4 * half + e] = acc[jq * 4 + e] * inv;
+    __builtin_amdgcn_wave_barrier();
+    // lane l: rows l / 8 + 8 k, columns 4 (l % 8) .. + 3
+    const int c4 = (lane & 7) * 4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int rl = (lane >> 3) + 8 * k;
+      if (rb * 32 + rl >= rows) continue;
+      floatx4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = tile[wave][rl][c4 + e];
+      *reinterpret_cast<floatx4_t *>(out + ((int64_t)b * rows + rb * 32 + rl) * R + cb * 32 + c4) = v;
+    }
+    return;
   }
   if (half == 0) {
     wave_mx[wave][n] = mx;
@@ -1294,18 +1321,32 @@ __global__ __launch_bounds__(256) void k_decode_narrow(
   } while (next_seq < batch);
 }
 
+// Slots of the longest sequence: the pieces its tokens reach (plan_round).
+int64_t max_slots(const DecodeArgs &a, int32_t r) {
+  const int64_t seg = decode_mfma_seg_tokens(a.rows, r, a.dr);
+  int64_t total = 0, longest = 0;
+  for (int32_t i = 0; i < a.batch; ++i) {
+    const int64_t n = (int64_t)a.cache->h_lens[i] + a.pending;
+    total += n + seg;
+    longest = std::max(longest, n);
+  }
+  const int64_t piece = std::max<int64_t>(kTok, (total + a.blocks - 1) / a.blocks);
+  return longest / piece + 1;
+}
+
 template <int R>
 qmla_status launch_merge(const DecodeArgs &a, hipStream_t stream) {
   const int row_blocks = (a.rows + 31) / 32;
-  // Slots per sequence (about blocks / batch) decide.  More than 16, past the
-  // plain merge's one round trip: 16 heads, 1 x 4097 27.6 -> 15.9 us (the whole
+  // The longest sequence's slots decide.  More than 16, past the plain merge's
+  // one round trip: 16 heads, 1 x 4097 27.6 -> 15.9 us (the whole
   // call), 1 x 32768 79.0 -> 30.4, 4 x 1000 16.7 -> 13.0.  From 9 slots where the
   // grid is at most two blocks per CU: 128 heads, 8 x 1000 27.0 -> 25.1, but 16 x
   // 4000 44.0 -> 45.1.  At fewer the LDS round is not won back: 1 x 40 11.4 ->
   // 12.8, 16 x 100 12.4 -> 13.6.
-  if (a.blocks > (a.batch * row_blocks <= 32 ? 8 : 16) * a.batch) {
+  const int few = a.batch * row_blocks <= 32 ? 8 : 16;
+  if (max_slots(a, R) > few) {
     k_decode_merge_split<R><<<dim3((unsigned)(a.batch * row_blocks), R / 32), dim3(kMergeWaves * 64), 0, stream>>>(
-        a.rows, row_blocks, a.seq_info, (const uint16_t *)a.part_o, a.part_lse, a.out, a.out_lse,
+        a.rows, row_blocks, few, a.seq_info, (const uint16_t *)a.part_o, a.part_lse, a.out, a.out_lse,
         a.advance ? a.cache->d_lens : nullptr, a.pending, a.batch);
     QMLA_LAUNCH_CHECK("k_decode_merge_split");
     return QMLA_OK;
