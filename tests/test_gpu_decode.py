@@ -419,3 +419,26 @@ def test_decode_bf16_one_piece_per_compute_unit_at_rank_512(qmla_gpu, rows_m):
     out, _ = run(q, cache, ql, qr, 0.06)
     ref, _ = O.decode_absorbed(ql, qr, rows, offs, np.asarray(lens, np.int32), 0.06)
     assert rel_err(out, ref) < TOL_BF16
+
+
+@pytest.mark.parametrize("r,dr,rows_m,k", [(512, 64, 16, 4), (512, 64, 128, 4), (512, 64, 40, 20), (64, 16, 48, 4),
+                                           (128, 32, 33, 9), (512, 64, 128, 64)])
+def test_decode_bf16_merges_one_long_sequence_among_short(qmla_gpu, r, dr, rows_m, k):
+    """One sequence of many partial slots among empty ones and ones of few:
+    each is merged by its own count, on grids on both sides of the line from
+    which every sequence takes the plain merge (64 x 4 + 1 sequences)."""
+    q = qmla_gpu
+    lens = np.asarray([0, 2500] + [7, 0, 40, 333] * k, np.int32)
+    cache, rows, offs = make_cache(q, lens, r, dr, q.BF16, 1970 + k)
+    b, n = len(lens), 10
+    ql, qr = O.normal((b, rows_m, r), 1971), O.normal((b, rows_m, dr), 1972)
+    ref, rlse = O.decode_absorbed(ql[:n], qr[:n], rows, offs[:n], lens[:n], 0.06)
+    live = lens[:n] > 0
+    for splits in (0, b, 256):
+        out, lse = run(q, cache, ql, qr, 0.06, splits=splits)
+        assert np.isfinite(out).all() and np.all(out[lens == 0] == 0) and np.all(np.isneginf(lse[lens == 0]))
+        assert rel_err(out[:n], ref) < TOL_BF16
+        np.testing.assert_allclose(lse[:n][live], rlse[live], atol=2e-2)
+        last, l_lse = O.decode_absorbed(ql[-2:], qr[-2:], rows, offs[-2:], lens[-2:], 0.06)
+        assert rel_err(out[-2:], last) < TOL_BF16
+        np.testing.assert_allclose(lse[-2:], l_lse, atol=2e-2)
