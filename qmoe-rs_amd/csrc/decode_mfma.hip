@@ -1321,12 +1321,13 @@ __global__ __launch_bounds__(256) void k_decode_narrow(
   } while (next_seq < batch);
 }
 
-// Slots of the longest sequence: the pieces its tokens reach (plan_round).
+// Slots of the longest sequence: the pieces its tokens reach (plan_round).  The
+// host's lengths include a layer step's pending tokens.
 int64_t max_slots(const DecodeArgs &a, int32_t r) {
   const int64_t seg = decode_mfma_seg_tokens(a.rows, r, a.dr);
   int64_t total = 0, longest = 0;
   for (int32_t i = 0; i < a.batch; ++i) {
-    const int64_t n = (int64_t)a.cache->h_lens[i] + a.pending;
+    const int64_t n = a.cache->h_lens[i];
     total += n + seg;
     longest = std::max(longest, n);
   }
