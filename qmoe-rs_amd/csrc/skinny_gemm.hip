@@ -93,8 +93,10 @@ __device__ __forceinline__ int64_t packed_b_offset(int m, int64_t k) {
 // operands (the weights' hi halves and bf16(x), one MFMA per step).
 constexpr int kXF32 = 0, kXPacked = 1, kXSum = 2;
 
+// Eight waves keep to 128 registers, so that two blocks fit a compute unit (the
+// packed and summed forms do by themselves).
 template <int NW, int XM, bool B16>
-__global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, LatentRowsArgs rows,
+__global__ __launch_bounds__(NW * 64, NW == 8 && XM == kXF32 ? 4 : 1) void k_skinny_gemm(SkinnyGemmArgs a, LatentRowsArgs rows,
                                                          int n_rows) {
   // LDS: the waves' partial tiles, or a latent row block's row
   extern __shared__ float smem[];
@@ -204,16 +206,25 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
   };
   // Eight waves: one pair per thread, requested ahead of the weights and
   // turned into the rotation under their latency (one user's step 45.4 -> 44.1
-  // us; after the reduction these were two more round trips).
-  constexpr bool kAhead = NW == 8;
+  // us; after the reduction these were two more round trips).  They wait in the
+  // thread's own LDS slot {b0, b1, cos, sin}: in registers they cost products of
+  // more tiles than units the second block per unit (hidden 5120, 128 heads, one
+  // user: q_proj | kv_a 87.7 us without them, 92.9 held in registers, 87.8 here).
+  constexpr bool kAhead = NW == 8 && XM == kXF32;  // as q_proj | kv_a runs
+  const bool pre_on = kAhead && a.mode == kSkinnyQkv;
+  floatx4_t *slot = reinterpret_cast<floatx4_t *>(smem + NW * 16 * 64) + threadIdx.x;
   Pre ahead{};
-  float cs_a = 0.f, sn_a = 0.f;
-  if constexpr (kAhead) ahead = prefetch(threadIdx.x);
+  if constexpr (kAhead)
+    if (pre_on) ahead = prefetch(threadIdx.x);
   // two chunks in flight: the loads of chunk i + 1 go out before the MFMAs
   // of chunk i
   load(0, 0);
   if constexpr (kAhead)
-    if (a.mode == kSkinnyQkv) rope_cs(ahead.pos * ahead.freq, a.mscale, cs_a, sn_a);
+    if (pre_on) {
+      float cs, sn;
+      rope_cs(ahead.pos * ahead.freq, a.mscale, cs, sn);
+      *slot = floatx4_t{ahead.b0, ahead.b1, cs, sn};
+    }
   int s0 = 0;
   for (; s0 + 2 * kChunk < steps; s0 += 2 * kChunk) {
     load(1, s0 + kChunk);
@@ -235,7 +246,13 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
   // epilogue over pairs (j, j + 1), j even: adjacent outputs of one token
   for (int e = threadIdx.x; e < 8 * 64; e += NW * 64) {
     const int j = 2 * (e >> 6), l = e & 63;
-    const Pre pre = kAhead ? ahead : prefetch(e);
+    floatx4_t pre = {0.f, 0.f, 0.f, 0.f};
+    if (pre_on) {
+      pre = *slot;
+    } else {
+      const Pre p = prefetch(e);
+      pre = floatx4_t{p.b0, p.b1, p.pos, p.freq};
+    }
     float v0 = 0.f, v1 = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
@@ -246,8 +263,8 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
     const int n = n0 + 8 * (j >> 2) + 4 * (l >> 5) + (j & 3);  // even
     if (m >= a.M || n >= a.N) continue;
     if (bias) {
-      v0 += pre.b0;
-      v1 += pre.b1;
+      v0 += pre[0];
+      v1 += pre[1];
     }
     if (a.mode == kSkinnyFinal) {
       float *y = a.y + z * a.sy + grp * a.sgrp + (int64_t)m * a.ldy + n;
@@ -286,8 +303,8 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_gemm(SkinnyGemmArgs a, Laten
       // interleaved pair (2p, 2p + 1) of q_rope (src/model.rs:70-84); the
       // rotation is linear, so each K-half is rotated on its own
       const int p = (d - a.dn) >> 1;
-      float cs = cs_a, sn = sn_a;
-      if constexpr (!kAhead) rope_cs(pre.pos * pre.freq, a.mscale, cs, sn);
+      float cs = pre[2], sn = pre[3];
+      if constexpr (!kAhead) rope_cs(pre[2] * pre[3], a.mscale, cs, sn);
       float *y = (grp ? a.q_rope1 : a.q_rope) + ((int64_t)mg * a.heads + hd) * a.dr + 2 * p;
       y[0] = v0 * cs - v1 * sn;
       y[1] = v1 * cs + v0 * sn;
@@ -354,7 +371,8 @@ qmla_status launch_skinny_gemm(const SkinnyGemmArgs &a, hipStream_t stream,
   SkinnyGemmArgs args = a;
   args.groups = G;
   dim3 grid((unsigned)((a.N + 31) / 32 * G + extra), (unsigned)a.Z);
-  const size_t lds = std::max(sizeof(float) * nw * 16 * 64,
+  // partial tiles and, with eight waves, the epilogue operands of each pair
+  const size_t lds = std::max(sizeof(float) * (nw * 16 * 64 + (nw == 8 ? 4 * 512 : 0)),
                               rows ? latent_row_lds_bytes(rows->r, rows->dr) : 0);
   if (a.x_packed) QMLA_REQUIRE(a.Z == 1, QMLA_ERR_SHAPE, "packed activations need Z = 1");
   auto go2 = [&](auto xm, auto b16) {
