@@ -416,7 +416,7 @@ int moe_grouped_max_tiles(int P, int E) { return P / kGroupTok + E; }
 
 bool moe_grouped_supported(const qmla_moe_config &c, int32_t T) {
   const int64_t P = (int64_t)T * c.top_k, H = c.hidden_dim, I = c.intermediate_dim;
-  return P >= (int64_t)kGroupedMinPairs * c.num_experts && H <= kGroupedMaxK && I <= kGroupedMaxK &&
+  return P >= moe_grouped_min_pairs(c.num_experts) && H <= kGroupedMaxK && I <= kGroupedMaxK &&
          route_lds_bytes(c.num_experts, c.hidden_dim) <= 96 * 1024 &&
          P * std::max(H, I) * 4 < (int64_t)1 << 32 && H * I / 4 < (int64_t)1 << 31;
 }

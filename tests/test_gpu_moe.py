@@ -287,3 +287,33 @@ def test_moe_grouped_nonfinite_and_zero_tokens(qmla_gpu):
     assert np.isnan(out[2]).all() and np.all(out[69] == 0)
     keep = [i for i in range(69) if i != 2]
     assert rel_err(out[keep], ref[keep]) < 2e-6
+
+
+@pytest.mark.parametrize("E,k,H,I,T", [
+    (1, 1, 128, 128, 383), (1, 1, 128, 128, 384), (2, 2, 128, 128, 193), (8, 2, 384, 640, 159), (8, 2, 384, 640, 161),
+    (5, 3, 1408, 2176, 107), (4, 4, 4224, 256, 81), (31, 4, 256, 384, 79), (31, 4, 256, 384, 80), (32, 4, 256, 384, 64)])
+def test_moe_forward_around_the_grouped_line(qmla_gpu, E, k, H, I, T):
+    """The last sizes of the GEMV and the first of the grouped path, which few
+    experts take from 320 pairs in all (384 below four experts), with the grouped
+    path's remainders (32 pairs, four tokens, row blocks).  Bound as above."""
+    q = qmla_gpu
+    W = O.random_moe_weights(E, k, H, I, 7700 + H + T)
+    xs = O.normal((T, H), 7800 + T)
+    out, idx, wts = moe_layer(q, W).forward(xs, return_routing=True)
+    ref, ridx, rw = O.moe_forward(W, xs, return_routing=True)
+    np.testing.assert_array_equal(idx, ridx)
+    np.testing.assert_allclose(wts, rw, rtol=1e-4, atol=1e-7)
+    assert rel_err(out, ref) < (8e-6 if T * k < (384 if E < 4 else 320) else 2e-6)
+
+
+def test_moe_grouped_nonfinite_and_zero_tokens_among_many(qmla_gpu):
+    """As above at a size that few experts group."""
+    q = qmla_gpu
+    W = O.random_moe_weights(4, 2, 256, 256, 43)
+    xs = O.normal((170, 256), 44)
+    ref = O.moe_forward(W, xs)
+    xs[2, 5], xs[9, 0], xs[169] = np.nan, np.inf, 0.0
+    out = moe_layer(q, W).forward(xs)
+    assert np.isnan(out[[2, 9]]).all() and np.all(out[169] == 0)
+    keep = [i for i in range(169) if i not in (2, 9)]
+    assert rel_err(out[keep], ref[keep]) < 2e-6
