@@ -243,7 +243,7 @@ def test_moe_forward_skewed_routing(qmla_gpu, H, I):
     (3, 2, 4224, 4352, 2), (8, 2, 640, 1000, 11), (2, 1, 256, 256, 15)])
 def test_moe_gemv_edges(qmla_gpu, E, k, H, I, T):
     """Fewer than eight pairs per expert: the GEMV path with its weights
-    requested before and after the bins are known (one pair per two experts),
+    requested before and after the bins are known (one pair per expert),
     bins of several tiles, row blocks past the last row, several slabs of K and
     a per-row down product.  The sums are exact integers here; the oracle's four
     f32 running sums of K / 4 <= 1088 products round by about 1088^0.5 2^-24 =
@@ -291,11 +291,14 @@ def test_moe_grouped_nonfinite_and_zero_tokens(qmla_gpu):
 
 @pytest.mark.parametrize("E,k,H,I,T", [
     (1, 1, 128, 128, 383), (1, 1, 128, 128, 384), (2, 2, 128, 128, 193), (8, 2, 384, 640, 159), (8, 2, 384, 640, 161),
-    (5, 3, 1408, 2176, 107), (4, 4, 4224, 256, 81), (31, 4, 256, 384, 79), (31, 4, 256, 384, 80), (32, 4, 256, 384, 64)])
-def test_moe_forward_around_the_grouped_line(qmla_gpu, E, k, H, I, T):
+    (5, 3, 1408, 2176, 107), (4, 4, 4224, 256, 81), (31, 4, 256, 384, 79), (31, 4, 256, 384, 80), (32, 4, 256, 384, 64),
+    (16, 1, 256, 512, 15), (16, 1, 256, 512, 16), (32, 4, 2048, 1408, 7), (32, 4, 2048, 1408, 8)])
+def test_moe_forward_around_its_lines(qmla_gpu, E, k, H, I, T):
     """The last sizes of the GEMV and the first of the grouped path, which few
     experts take from 320 pairs in all (384 below four experts), with the grouped
-    path's remainders (32 pairs, four tokens, row blocks).  Bound as above."""
+    path's remainders (32 pairs, four tokens, row blocks); and GEMV calls around
+    one pair per expert, from where the weights are requested at once.  Bounds as
+    above."""
     q = qmla_gpu
     W = O.random_moe_weights(E, k, H, I, 7700 + H + T)
     xs = O.normal((T, H), 7800 + T)
