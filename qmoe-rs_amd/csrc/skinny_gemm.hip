@@ -93,10 +93,9 @@ __device__ __forceinline__ int64_t packed_b_offset(int m, int64_t k) {
 // operands (the weights' hi halves and bf16(x), one MFMA per step).
 constexpr int kXF32 = 0, kXPacked = 1, kXSum = 2;
 
-// Eight waves keep to 128 registers, so that two blocks fit a compute unit (the
-// packed and summed forms do by themselves).
+// Eight waves keep to 128 registers, so that two blocks fit a compute unit.
 template <int NW, int XM, bool B16>
-__global__ __launch_bounds__(NW * 64, NW == 8 && XM == kXF32 ? 4 : 1) void k_skinny_gemm(SkinnyGemmArgs a, LatentRowsArgs rows,
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 4 : 1) void k_skinny_gemm(SkinnyGemmArgs a, LatentRowsArgs rows,
                                                          int n_rows) {
   // LDS: the waves' partial tiles, or a latent row block's row
   extern __shared__ float smem[];
@@ -209,9 +208,10 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && XM == kXF32 ? 4 : 1) void k_ski
   // us; after the reduction these were two more round trips).  They wait in the
   // thread's own LDS slot {b0, b1, cos, sin}: in registers they cost products of
   // more tiles than units the second block per unit (hidden 5120, 128 heads, one
-  // user: q_proj | kv_a 87.7 us without them, 92.9 held in registers, 87.8 here).
-  constexpr bool kAhead = NW == 8 && XM == kXF32;  // as q_proj | kv_a runs
-  const bool pre_on = kAhead && a.mode == kSkinnyQkv;
+  // user: q_proj | kv_a 87.7 us without them, 92.9 held in registers, 87.6 here;
+  // o_proj 72.3, 76.8 and 72.6).
+  constexpr bool kAhead = NW == 8 && XM != kXSum;
+  const bool pre_on = kAhead && (bias || a.mode == kSkinnyQkv);
   floatx4_t *slot = reinterpret_cast<floatx4_t *>(smem + NW * 16 * 64) + threadIdx.x;
   Pre ahead{};
   if constexpr (kAhead)
@@ -221,8 +221,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && XM == kXF32 ? 4 : 1) void k_ski
   load(0, 0);
   if constexpr (kAhead)
     if (pre_on) {
-      float cs, sn;
-      rope_cs(ahead.pos * ahead.freq, a.mscale, cs, sn);
+      float cs = 0.f, sn = 0.f;
+      if (a.mode == kSkinnyQkv) rope_cs(ahead.pos * ahead.freq, a.mscale, cs, sn);
       *slot = floatx4_t{ahead.b0, ahead.b1, cs, sn};
     }
   int s0 = 0;
@@ -247,8 +247,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 && XM == kXF32 ? 4 : 1) void k_ski
   for (int e = threadIdx.x; e < 8 * 64; e += NW * 64) {
     const int j = 2 * (e >> 6), l = e & 63;
     floatx4_t pre = {0.f, 0.f, 0.f, 0.f};
-    if (pre_on) {
-      pre = *slot;
+    if constexpr (kAhead) {
+      if (pre_on) pre = *slot;
     } else {
       const Pre p = prefetch(e);
       pre = floatx4_t{p.b0, p.b1, p.pos, p.freq};
