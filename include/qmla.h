@@ -290,13 +290,18 @@ QMLA_API qmla_status qmla_decode_workspace_bytes_splits(const qmla_decode_dims *
 /* Allocation-free form of qmla_decode_absorbed.  It has no counterpart in
  * the reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc).  Same arguments, results and errors as qmla_decode_absorbed,
+ * hipMalloc).  Same arguments and errors as qmla_decode_absorbed,
  * without the workspace: the split partials live in a static device array
  * of QMLA_DECODE_NOALLOC_SCRATCH_BYTES per GPU, held from the library's
- * first use of that GPU until the process ends.  A call whose workspace
- * (qmla_decode_workspace_bytes) would exceed that size returns
- * QMLA_ERR_UNSUPPORTED before anything is launched; the 128-head,
- * batch-64 decode over 256 compute units needs 40 MiB.  The call allocates
+ * first use of that GPU until the process ends.  Where that array holds the
+ * partials of qmla_decode_absorbed's own split (its workspace is then at most
+ * that size, or more only for the sake of calls with fewer rows or sequences),
+ * the results are the same bits.  Where it does not, the call runs
+ * with pieces of 128 tokens: on a bf16 cache the partials then round
+ * elsewhere, and results agree within the bf16 tolerance.  A call whose
+ * pieces of 128 tokens need more returns QMLA_ERR_UNSUPPORTED before
+ * anything is launched; the 128-head, batch-64 decode over 256 compute units
+ * needs 40 MiB.  The call allocates
  * nothing.  Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (other streams, other threads) race and must be
  * serialised by the caller. */

@@ -387,10 +387,12 @@ qmla_status validate_decode(const qmla_decode_dims *d, const qmla_kv_cache *c) {
 // minimum so that per-piece overhead (q load, partial write) stays small.
 // The MFMA plans count the virtual tokens they add per sequence: without them
 // 16 sequences of 100 tokens made 13 pieces of 444 virtual tokens, several
-// sequences to a piece.  f32: its 32-token tiles take 1.2 us each, so few
-// tokens go out one tile to a piece (278 tokens 27.8 us at 128 a piece, 14.1
-// at 32; 2222 tokens 28.3 and 17.3), for at most 32 rows and 64 sequences,
-// where the partials of 256 pieces stay below 22 MB.  bf16: two tiles (16
+// sequences to a piece.  f32: a lone block takes 3.6 us for a 32-token tile, so
+// few tokens go out one tile to a piece (278 tokens 24.0 us in 3 pieces, 13.6 in
+// 11; 8 x 278 27.8 in 18, 14.3 in 86), for at most 32 rows and 64 sequences: their
+// partials stay below 22 MB.  Beyond, pieces of 128 tokens without the virtual
+// ones are not the best (16 rows, 64 x 100 tokens 23.7 us, 65 x 100 41.8; the VALU
+// kernel took 200).  bf16: two tiles (16
 // heads, 128 / 64 / 32 tokens a piece: 1 x 200 14.1 / 12.5 / 12.5 us, 1 x 4097
 // 15.3 / 14.8 / 17.8, 16 x 100 14.5 / 12.5 / 12.6; 128 heads, 1 x 500 21.8 /
 // 19.1 / 18.8, 4 x 1000 24.0 / 23.1 / 26.0).  The VALU path keeps 128.

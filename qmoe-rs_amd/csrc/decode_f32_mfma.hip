@@ -2,10 +2,11 @@
 // (v_mfma_f32_16x16x4_f32: exact f32 products, f32 sums) for kv_lora_rank
 // 512 and rope 64.
 //
-// Bound: for a few users' contexts, the latency chain of one or two tiles per
-// block (lengths, first rows from HBM, merge launch); for long ones HBM: a
-// 32-token tile is 72 KB and 2,200 clocks of MFMA per SIMD, i.e. 34 B per
-// clock and CU.
+// Bound: for a few users' contexts, the latency chain of a block's first tile
+// (lengths, first rows from HBM, merge launch) and then its tiles one after the
+// other: a 32-token tile is 72 KB and 4,350 clocks of MFMA per SIMD (two waves of
+// 68 MFMAs of 32 clocks), 17 B per clock and CU.  A lone block takes 3.6 us a
+// tile, half of it MFMA; with 256 blocks 5.2 us, 3.6 TB/s.
 //
 // Split: one block of eight waves per piece of the concatenated tokens
 // (decode_plan.hpp) and 16 query rows.  Waves 0-3 take the first 16 tokens of
@@ -25,7 +26,7 @@
 // 8 users of 300-4000 tokens, 16 heads (20.5K tokens, 47 MB): 26 us, decode
 // and merge, 1.8 TB/s, against 304 us with the VALU kernel of decode.hip, which
 // reads the cache once per query row; 8 x 4000 tokens 32 us, 2.3 TB/s.  Relative
-// error against 64 bits 3.3e-7 (VALU kernel 5.1e-7).
+// error against 64 bits 3.1e-7 to 3.3e-7 (VALU kernel 5.2e-7 to 5.6e-7).
 
 #include "decode_plan.hpp"
 #include "mfma_pipe.hpp"

@@ -248,8 +248,9 @@ def test_prefill_f32_unaligned_tensors(qmla_gpu):
 
 def test_prefill_f32_infinite_last_value(qmla_gpu):
     """An infinite value in the last key's column 5 makes that column of the
-    last row infinite (not NaN) and no other, though the last key tile is
-    partial."""
+    last row infinite (not NaN), though the last key tile is partial.  Other
+    columns are untouched; column 5 stays finite in the rows of other tiles,
+    while rows 32..39, which share the last row's tile, hold 0 x inf there."""
     arrs = inputs(1, 1, 41, 41, 128, 64, 128, 1, 780)
     ref = O.fused_prefill_attn(*arrs, 0.1, True)
     arrs[4][0, 0, 40, 5] = np.inf
