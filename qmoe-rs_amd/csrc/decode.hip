@@ -425,15 +425,30 @@ int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t
   return (int32_t)std::min<int64_t>(blocks, kMaxPlanBlocks);
 }
 
-// Pieces the bf16 plan launches of the `blocks` it may: pieces of two to four
-// tiles become whole tiles, since cut at 67 tokens some hold three tiles and
+// Pieces the bf16 plan launches of the `blocks` it may.  Above 128 rows each
+// piece is a block per 128 rows, and at rank 512 a compute unit holds one block:
+// no more pieces than one round takes (256 rows, 4 x 4000 tokens 50.4 -> 33.8 us,
+// 64 x 1000 88 -> 64, 64 x 4000 200 -> 161).  Then pieces of two to four tiles become whole tiles, since cut at 67 tokens some hold three tiles and
 // the rest two, with more partials to merge than pieces of three (16 heads, 4 x
-// 4000: 18.8 -> 16.7 us).
-int32_t whole_tile_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t blocks) {
+// 4000: 18.8 -> 16.7 us).  Above 64 rows, where a piece's partial is larger than
+// the tokens of two tiles, a sequence of more than 80 pieces takes three: its
+// merge is the longer part (128 heads, 8192 + 15 x 10 tokens 40.4 -> 35.7 us; with
+// up to 24 pieces per sequence two stay better, 8 x 1000 25.2 us against 26.3).
+int32_t launch_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t blocks) {
+  if (d->rows > 128 && d->kv_lora_rank == 512) {
+    int cus = device_cu_count();
+    if (cus <= 0) cus = 256;
+    blocks = std::min(blocks, std::max(1, cus / ((d->rows + 127) / 128)));
+  }
   int64_t total = (int64_t)d->batch * decode_mfma_seg_tokens(d->rows, d->kv_lora_rank, d->rope_dim);
-  for (int32_t i = 0; i < d->batch; ++i) total += c->h_lens[i];
-  const int64_t tiles = (total + 32LL * blocks - 1) / (32LL * blocks);
+  int32_t longest = 0;
+  for (int32_t i = 0; i < d->batch; ++i) {
+    total += c->h_lens[i];
+    longest = std::max(longest, c->h_lens[i]);
+  }
+  int64_t tiles = (total + 32LL * blocks - 1) / (32LL * blocks);
   if (tiles < 2 || tiles > 4) return blocks;
+  if (d->rows > 64 && longest > 80 * 64) tiles = std::max<int64_t>(tiles, 3);
   return (int32_t)std::max<int64_t>(1, std::min<int64_t>(blocks, (total + 32 * tiles - 1) / (32 * tiles)));
 }
 
@@ -509,7 +524,7 @@ qmla_status qmla::decode_launch(const qmla_decode_dims *d, const qmla_kv_cache *
   a.seq_info = reinterpret_cast<int2 *>(ws);
   a.part_o = reinterpret_cast<float *>(static_cast<char *>(ws) + lay.part_o_off);
   a.part_lse = reinterpret_cast<float *>(static_cast<char *>(ws) + lay.part_lse_off);
-  a.blocks = mfma && splits <= 0 ? whole_tile_blocks(d, c, blocks) : blocks;
+  a.blocks = mfma && splits <= 0 ? launch_blocks(d, c, blocks) : blocks;
   a.pending = pending;
   a.advance = advance;
   if (mfma) return launch_decode_mfma(a, s);  // decode + merge

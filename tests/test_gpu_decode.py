@@ -442,3 +442,22 @@ def test_decode_bf16_merges_one_long_sequence_among_short(qmla_gpu, r, dr, rows_
         last, l_lse = O.decode_absorbed(ql[-2:], qr[-2:], rows, offs[-2:], lens[-2:], 0.06)
         assert rel_err(out[-2:], last) < TOL_BF16
         np.testing.assert_allclose(lse[-2:], l_lse, atol=2e-2)
+
+
+@pytest.mark.parametrize("r,dr,rows_m", [(512, 64, 65), (512, 64, 128), (512, 64, 129), (512, 64, 300), (512, 64, 520),
+                                         (64, 16, 160), (128, 32, 130)])
+def test_decode_bf16_many_rows_and_a_long_sequence(qmla_gpu, r, dr, rows_m):
+    """Several blocks of 128 rows per piece, whose pieces fit one round of the
+    device, and a sequence past 80 pieces of 64 tokens, which takes pieces of
+    three tiles, beside short and empty ones."""
+    q = qmla_gpu
+    lens = [5200, 0, 33, 700, 1, 64]
+    cache, rows, offs = make_cache(q, lens, r, dr, q.BF16, 1980 + rows_m, cap_extra=1)
+    b = len(lens)
+    ql, qr = O.normal((b, rows_m, r), 1981), O.normal((b, rows_m, dr), 1982)
+    ref, rlse = O.decode_absorbed(ql, qr, rows, offs, np.asarray(lens, np.int32), 0.06)
+    live = np.asarray(lens) > 0
+    out, lse = run(q, cache, ql, qr, 0.06)
+    assert rel_err(out, ref) < TOL_BF16
+    assert np.all(out[~live] == 0) and np.all(np.isneginf(lse[~live]))
+    np.testing.assert_allclose(lse[live], rlse[live], atol=2e-2)
