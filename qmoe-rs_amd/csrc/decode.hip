@@ -430,7 +430,10 @@ int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t
 // no more pieces than one round takes (256 rows, 4 x 4000 tokens 50.4 -> 33.8 us,
 // 64 x 1000 88 -> 64, 64 x 4000 200 -> 161).  Then pieces of two to four tiles become whole tiles, since cut at 67 tokens some hold three tiles and
 // the rest two, with more partials to merge than pieces of three (16 heads, 4 x
-// 4000: 18.8 -> 16.7 us).  Above 64 rows, where a piece's partial is larger than
+// 4000: 18.8 -> 16.7 us).  At 33 .. 64 rows many sequences have too few slots each
+// to gain (48 rows, whole tiles / as cut: 10 x 2000 24.4 / 25.4, 2 x 10000 27.5 /
+// 29.0, but 16 x 1000 26.8 / 26.1, 32 x 500 27.5 / 25.5, 64 x 200 28.3 / 24.8, 100 x
+// 200 34.6 / 32.8).  Above 64 rows, where a piece's partial is larger than
 // the tokens of two tiles, a sequence of more than 80 pieces takes three: its
 // merge is the longer part (128 heads, 8192 + 15 x 10 tokens 40.4 -> 35.7 us; with
 // up to 24 pieces per sequence two stay better, 8 x 1000 25.2 us against 26.3).
@@ -448,6 +451,7 @@ int32_t launch_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t
   }
   int64_t tiles = (total + 32LL * blocks - 1) / (32LL * blocks);
   if (tiles < 2 || tiles > 4) return blocks;
+  if (d->rows > 32 && d->rows <= 64 && d->batch > 15) return blocks;
   if (d->rows > 64 && longest > 80 * 64) tiles = std::max<int64_t>(tiles, 3);
   return (int32_t)std::max<int64_t>(1, std::min<int64_t>(blocks, (total + 32 * tiles - 1) / (32 * tiles)));
 }

@@ -1342,14 +1342,15 @@ qmla_status launch_merge(const DecodeArgs &a, hipStream_t stream) {
   // one round trip: 16 heads, 1 x 4097 27.6 -> 15.9 us (the whole
   // call), 1 x 32768 79.0 -> 30.4, 4 x 1000 16.7 -> 13.0.  From 9 slots where the
   // grid is at most two blocks per CU: 128 heads, 8 x 1000 27.0 -> 25.1, but 16 x
-  // 4000 44.0 -> 45.1.  At fewer the LDS round is not won back: 1 x 40 11.4 ->
-  // 12.8, 16 x 100 12.4 -> 13.6.
+  // 4000 44.0 -> 45.1.  From 5 where it is at most one: 48 rows, 1 x 500 17.3 -> 16.3,
+  // 4 x 450 17.8 -> 16.8, 128 heads, 1 x 400 19.9 -> 18.9.  At fewer the LDS round is
+  // not won back: 1 x 40 11.4 -> 12.8, 16 x 100 12.4 -> 13.6.
   // One long sequence among many pays once its slots outweigh the blocks that
   // have nothing to do, about 6.6 ns per (sequence, row block) against 0.2 us
   // per slot: 128 heads, 8192 + 255 x 50 tokens (21 slots) 60.9 us plain, 66.5
   // split; 32768 + 255 x 50 (66 slots) 82.2 and 78.6.
   const int64_t tiles = (int64_t)a.batch * row_blocks;
-  const int few = tiles <= 32 ? 8 : 16;
+  const int few = tiles <= 16 ? 4 : tiles <= 32 ? 8 : 16;
   if (max_slots(a, R) > few + (tiles <= 32 ? 0 : tiles / 32)) {
     k_decode_merge_split<R><<<dim3((unsigned)(a.batch * row_blocks), R / 32), dim3(kMergeWaves * 64), 0, stream>>>(
         a.rows, row_blocks, few, a.seq_info, (const uint16_t *)a.part_o, a.part_lse, a.out, a.out_lse,
