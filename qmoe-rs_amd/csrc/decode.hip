@@ -436,7 +436,10 @@ int32_t choose_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t
 // 200 34.6 / 32.8).  Above 64 rows, where a piece's partial is larger than
 // the tokens of two tiles, a sequence of more than 80 pieces takes three: its
 // merge is the longer part (128 heads, 8192 + 15 x 10 tokens 40.4 -> 35.7 us; with
-// up to 24 pieces per sequence two stay better, 8 x 1000 25.2 us against 26.3).
+// up to 24 pieces per sequence two stay better, 8 x 1000 25.2 us against 26.3).  One
+// tile in all is one piece (1 x 16 9.04 -> 8.81 us); several are not held to their
+// number, since the cuts would fall worse (4 x 100 11.2 / 12.2, 8 x 16 of rank 64
+// 7.3 / 9.0).
 int32_t launch_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t blocks) {
   if (d->rows > 128 && d->kv_lora_rank == 512) {
     int cus = device_cu_count();
@@ -449,6 +452,7 @@ int32_t launch_blocks(const qmla_decode_dims *d, const qmla_kv_cache *c, int32_t
     total += c->h_lens[i];
     longest = std::max(longest, c->h_lens[i]);
   }
+  if (d->batch == 1 && longest <= 32) return 1;
   int64_t tiles = (total + 32LL * blocks - 1) / (32LL * blocks);
   if (tiles < 2 || tiles > 4) return blocks;
   if (d->rows > 32 && d->rows <= 64 && d->batch > 15) return blocks;
