@@ -293,7 +293,8 @@ bool split_gemm_supported(int N, int K);
 // The reduction of a.ksplit planes of partial sums, bias and epilogue.
 qmla_status launch_sg_reduce(const SplitGemmArgs &a, hipStream_t stream);
 // K slices the split GEMM uses for an M x N x K product (1 when its tiles
-// already fill the device), and the partial-sum bytes they need.
+// already fill the device), and the partial-sum bytes that products of up to M
+// rows need.
 int split_gemm_slices(int M, int N, int K);
 size_t split_gemm_part_bytes(int M, int N, int K);
 // Rows from which the split GEMM runs its 256 x 256 tiles, and below which

@@ -866,13 +866,19 @@ size_t decode_bytes_for(const qmla_layer *L, const qmla_kv_cache *c, int32_t bat
                         int32_t seq) {
   int cus = device_cu_count();
   if (cus <= 0) cus = 256;
-  const int32_t rows = seq * L->cfg.heads, r = L->cfg.kv_lora_rank, dr = L->cfg.qk_rope;
+  const int32_t all = seq * L->cfg.heads, r = L->cfg.kv_lora_rank, dr = L->cfg.qk_rope;
   const bool mfma = c->dtype == QMLA_BF16;
-  const int per_cu = mfma && decode_mfma_supported(rows, r, dr)
-                         ? decode_mfma_blocks_per_cu(rows, r, dr)
-                         : decode_f32_blocks_per_cu(r, dr);
-  const int32_t blocks = (int32_t)std::min<int64_t>((int64_t)cus * per_cu, kMaxPlanBlocks);
-  return decode_workspace_layout(batch, rows, r, blocks, mfma).total;
+  size_t most = 0;
+  // pieces per unit depend on the rows (up to 32, up to 64, more): the largest
+  // step of each class, so that the size serves fewer new tokens too
+  for (int32_t rows : {std::min(all, 32), std::min(all, 64), all}) {
+    const int per_cu = mfma && decode_mfma_supported(rows, r, dr)
+                           ? decode_mfma_blocks_per_cu(rows, r, dr)
+                           : decode_f32_blocks_per_cu(r, dr);
+    const int32_t blocks = (int32_t)std::min<int64_t>((int64_t)cus * per_cu, kMaxPlanBlocks);
+    most = std::max(most, decode_workspace_layout(batch, rows, r, blocks, mfma).total);
+  }
+  return most;
 }
 
 }  // namespace

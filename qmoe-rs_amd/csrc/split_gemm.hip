@@ -574,8 +574,15 @@ int split_gemm_slices(int M, int N, int K) {
 }
 
 size_t split_gemm_part_bytes(int M, int N, int K) {
-  const int s = split_gemm_slices(M, N, K);
-  return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+  size_t most = 0;
+  auto take = [&](int m) {
+    const int s = split_gemm_slices(m, N, K);
+    if (s > 1) most = std::max(most, (size_t)s * m * N * sizeof(float));
+  };
+  take(M);
+  // the slices change where another 128-row tile begins
+  for (int m = 128; m < std::min(M, kSplitGemmBigRows); m += 128) take(m);
+  return most;
 }
 
 namespace {

@@ -692,12 +692,10 @@ def test_layer_workspace_serves_fewer_tokens(qmla_gpu, dt, hidden, H, dn, dr, dv
     q = qmla_gpu
     layer = q.MlaLayer(O.MlaWeights.random(hidden, H, dn, dr, dv, r, seed=1950))
     cache = q.KVCache([512] * 200, r, dr, q.F32 if dt == "f32" else q.BF16)
-    short = [1, 7, 32, 33, 63, 64, 65, 66, 100, 126, 127]
-    for long in short + [128, 129, 140, 200, 300]:
-        pre, step = layer.prefill_workspace_bytes(cache, 1, long), layer.workspace_bytes(cache, 1, long)
-        for n in short:
-            if n < long:
-                assert layer.prefill_workspace_bytes(cache, 1, n) <= pre, (n, long)
-                assert layer.workspace_bytes(cache, 1, n) <= step, (n, long)
+    sizes = [1, 7, 8, 9, 16, 17, 32, 33, 63, 64, 65, 66, 100, 126, 127, 128, 129, 140, 200, 256, 257, 300, 512, 513, 600,
+             1024, 1025, 2048, 2049, 4095, 4096, 4097]
+    pre = [layer.prefill_workspace_bytes(cache, 1, n) for n in sizes]
+    both = [layer.workspace_bytes(cache, 1, n) for n in sizes]
+    assert pre == sorted(pre) and both == sorted(both)
     steps = [layer.workspace_bytes(cache, b, 1) for b in (1, 31, 32, 33, 63, 64, 65, 66, 100, 127, 128, 200)]
     assert steps == sorted(steps)
