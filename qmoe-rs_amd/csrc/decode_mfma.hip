@@ -1350,8 +1350,14 @@ qmla_status launch_merge(const DecodeArgs &a, hipStream_t stream) {
   // per slot: 128 heads, 8192 + 255 x 50 tokens (21 slots) 60.9 us plain, 66.5
   // split; 32768 + 255 x 50 (66 slots) 82.2 and 78.6.
   const int64_t tiles = (int64_t)a.batch * row_blocks;
-  const int few = tiles <= 16 ? 4 : tiles <= 32 ? 8 : 16;
-  if (max_slots(a, R) > few + (tiles <= 32 ? 0 : tiles / 32)) {
+  const int64_t line = tiles <= 16 ? 4 : tiles <= 32 ? 8 : 16 + tiles / 32;
+  if (max_slots(a, R) > line) {
+    // Beside a long sequence, those of up to 4 slots go to one wave; on a small
+    // grid none does, since the blocks are there (48 rows, 24 ragged sequences of
+    // up to 2000 tokens 31.1 us with 16 slots to one wave, 28.5 with 4; 128 heads,
+    // 99 of 50 beside 8192 44.7 with 4, 54.8 with none; 16 heads, 12 of 34-553 12.3
+    // with none, 12.8 with 4).
+    const int few = tiles <= 32 ? 0 : 4;
     k_decode_merge_split<R><<<dim3((unsigned)(a.batch * row_blocks), R / 32), dim3(kMergeWaves * 64), 0, stream>>>(
         a.rows, row_blocks, few, a.seq_info, (const uint16_t *)a.part_o, a.part_lse, a.out, a.out_lse,
         a.advance ? a.cache->d_lens : nullptr, a.pending, a.batch);
